@@ -18,7 +18,16 @@
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kTile = 2048;  // positions per scatter workgroup (8 per thread)
+constexpr int kTile = 2048;        // positions per count tile
+constexpr int kRows = 64;          // positions per scatter workgroup
+constexpr int kPlanThreads = 1024;
+constexpr int kPlanWaves = kPlanThreads / 64;
+// Up to this many count tiles (heads x tiles) the plan workgroup counts the
+// flags itself; beyond, admit_count_kernel does, in a launch before it.  Whole
+// call at 8 heads, counted by the plan / by the extra launch: 777 tokens (8
+// tiles) 10.8 / 11.6 us, 6100 (24) 12.8 / 12.8, 9001 (40) 15.3 / 13.9, 32768
+// (128) 28.1 / 21.6.
+constexpr int kPlanCounts = 24;
 
 struct AdmitArgs {
   const uint16_t* key;
@@ -46,69 +55,121 @@ struct AdmitArgs {
   int32_t* abort_flag;
 };
 
-// Copies `n` rows of D bf16 (src row pointers / dst pool rows from LDS lists)
-// with the whole workgroup, 16 bytes per thread per step.
-__device__ void copy_rows(const uint16_t* __restrict__ base, int64_t ss, const int* s_src, const int64_t* s_dst,
-                          int n, int D, uint16_t* __restrict__ dst_pool) {
-  const int chunks = D / 8;
-  for (int e = threadIdx.x; e < n * chunks; e += kThreads) {
-    const int r = e / chunks, c = e - r * chunks;
-    const u32x4_t v = *(const u32x4_t*)(base + (int64_t)s_src[r] * ss + c * 8);
-    *(u32x4_t*)(dst_pool + s_dst[r] * D + c * 8) = v;
+// Copies rows r < n of one K/V pair (source row src(r), pool row dst(r)) with
+// the whole workgroup, 16 bytes per thread and step.  Eight loads per thread
+// are requested before the first store: one load and one store at a time
+// waited for memory once per step (64 us of a 9001-token prompt's 75).
+template <typename Src, typename Dst>
+__device__ __forceinline__ void copy_rows2(const uint16_t* ka, const uint16_t* va, int64_t ss, int n, int D, Src src,
+                                           Dst dst, uint16_t* pool_k, uint16_t* pool_v) {
+  constexpr int U = 4;
+  const unsigned chunks = D / 8;
+  const unsigned total = n * chunks;
+  for (unsigned e0 = threadIdx.x; e0 < total; e0 += kThreads * U) {
+    u32x4_t k[U], v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const unsigned e = min(e0 + u * kThreads, total - 1);
+      const unsigned r = e / chunks;
+      const int64_t off = (int64_t)src(r) * ss + (e - r * chunks) * 8;
+      k[u] = *(const u32x4_t*)(ka + off);
+      v[u] = *(const u32x4_t*)(va + off);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const unsigned e = e0 + u * kThreads;
+      if (e >= total) break;
+      const unsigned r = e / chunks;
+      const int64_t off = dst(r) * D + (e - r * chunks) * 8;
+      *(u32x4_t*)(pool_k + off) = k[u];
+      *(u32x4_t*)(pool_v + off) = v[u];
+    }
   }
 }
 
+// Flags of one count tile of one head (prompts of many tiles only).
 __global__ __launch_bounds__(kThreads) void admit_count_kernel(AdmitArgs a) {
-  __shared__ int s_red[kThreads];
+  __shared__ int s_w[kThreads / 64];
   const int h = blockIdx.y, tile = blockIdx.x;
-  const int n_early = max(0, a.S - a.W);
-  const uint8_t* m = a.mask + (int64_t)h * a.m_sh;
-  int cnt = 0;
-  for (int p = tile * kTile + threadIdx.x; p < min(n_early, (tile + 1) * kTile); p += kThreads) cnt += m[p] != 0;
-  s_red[threadIdx.x] = cnt;
+  const int t = threadIdx.x;
+  const int lo = tile * kTile, hi = min(max(0, a.S - a.W), lo + kTile);
+  const int c = wave_sum_int(count_flags(a.mask + (int64_t)h * a.m_sh, lo, hi, t, kThreads));
+  if ((t & 63) == 0) s_w[t >> 6] = c;
   __syncthreads();
-  for (int off = kThreads / 2; off > 0; off >>= 1) {
-    if (threadIdx.x < off) s_red[threadIdx.x] += s_red[threadIdx.x + off];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) a.tile_cnt[h * a.ntiles + tile] = s_red[0];
+  if (t == 0) a.tile_cnt[h * a.ntiles + tile] = (s_w[0] + s_w[1]) + (s_w[2] + s_w[3]);
 }
 
-// One workgroup: per-head totals, capacity checks, page allocation in head
-// order (src/modeling_layers.py:1303-1331), block-table rows, lengths.
-__global__ __launch_bounds__(kThreads) void admit_plan_kernel(AdmitArgs a) {
-  __shared__ int s_tmp[kThreads];
+// One workgroup: per-head totals (with COUNT from the flags themselves),
+// capacity checks, page allocation in head order
+// (src/modeling_layers.py:1303-1331), block-table rows, lengths.  A wave
+// counts a tile in two 16-byte loads per lane and takes a head's tiles in one
+// scan of 64, so the launch waits on memory a few times whatever the prompt's
+// length (one thread per head walking its tiles and pages took a memory round
+// trip for each).
+template <bool COUNT>
+__global__ __launch_bounds__(kPlanThreads) void admit_plan_kernel(AdmitArgs a) {
+  __shared__ int s_cnt[COUNT ? kPlanCounts : 1];
   __shared__ int s_n[1024];
-  __shared__ int s_fail;
-  const int t = threadIdx.x;
-  if (t == 0) s_fail = 0;
-  __syncthreads();
+  __shared__ int s_pg[1024];
+  __shared__ int s_fail, s_total, s_nf;
+  const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+  const int n_early = max(0, a.S - a.W);
   const int n_loc = min(a.S, a.W);
   const int lb = a.W / a.page;
-  // per-head totals and within-head tile prefixes (one thread per head)
-  for (int h = t; h < a.H; h += kThreads) {
-    int run = 0;
-    for (int tl = 0; tl < a.ntiles; ++tl) {
-      a.tile_base[h * a.ntiles + tl] = run;
-      run += a.tile_cnt[h * a.ntiles + tl];
+  if (t == 0) {
+    s_fail = 0;
+    s_nf = *a.next_free;
+  }
+  if constexpr (COUNT) {
+    const int n = a.H * a.ntiles;
+    constexpr int U = 4;  // tiles whose loads a wave has in flight
+    for (int i0 = wid; i0 < n; i0 += kPlanWaves * U) {
+      int c[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int i = i0 + u * kPlanWaves;
+        const int h = i / a.ntiles, lo = (i - h * a.ntiles) * kTile;
+        c[u] = i < n ? count_flags(a.mask + (int64_t)h * a.m_sh, lo, min(n_early, lo + kTile), lane, 64) : 0;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int s = wave_sum_int(c[u]);
+        if (lane == 0 && i0 + u * kPlanWaves < n) s_cnt[i0 + u * kPlanWaves] = s;
+      }
     }
-    s_n[h] = run;
-    if (run > 0 && (n_loc + run > a.max_tokens_per_head || lb + (run + a.page - 1) / a.page > a.max_pages))
-      atomicOr(&s_fail, 1);
+    __syncthreads();
+  }
+  for (int h = wid; h < a.H; h += kPlanWaves) {
+    int run = 0;
+    for (int t0 = 0; t0 < a.ntiles; t0 += 64) {
+      const int tl = t0 + lane;
+      int c = 0;
+      if (tl < a.ntiles) c = COUNT ? s_cnt[h * a.ntiles + tl] : a.tile_cnt[h * a.ntiles + tl];
+      const int incl = wave_incl_scan(c, lane);
+      if (tl < a.ntiles) a.tile_base[h * a.ntiles + tl] = run + incl - c;
+      run += __builtin_amdgcn_readlane(incl, 63);
+    }
+    if (lane == 0) s_n[h] = run;
   }
   __syncthreads();
-  // exclusive scan of pages over heads (H <= 1024, one pass per 256 heads)
-  const int nf = *a.next_free;
-  int carry = 0;
-  for (int h0 = 0; h0 < a.H; h0 += kThreads) {
-    const int h = h0 + t;
-    const int pages = h < a.H ? (s_n[h] + a.page - 1) / a.page : 0;
-    int total = 0;
-    const int excl = block_exclusive_scan_256(pages, s_tmp, &total);
-    if (h < a.H) a.head_row[h] = (int64_t)(nf + carry + excl) * a.page;
-    carry += total;
+  // first page of each head, relative to the bump pointer, and the checks
+  if (wid == 0) {
+    int carry = 0, bad = 0;
+    for (int h0 = 0; h0 < a.H; h0 += 64) {
+      const int h = h0 + lane;
+      const int n = h < a.H ? s_n[h] : 0;
+      const int pages = (n + a.page - 1) / a.page;
+      if (n > 0 && (n_loc + n > a.max_tokens_per_head || lb + pages > a.max_pages)) bad = 1;
+      const int incl = wave_incl_scan(pages, lane);
+      if (h < a.H) s_pg[h] = carry + incl - pages;
+      carry += __builtin_amdgcn_readlane(incl, 63);
+    }
+    bad = __builtin_amdgcn_ballot_w64(bad != 0) != 0;
+    if (lane == 0) {
+      s_total = carry;
+      if (bad || (int64_t)s_nf + carry > a.total_pages) s_fail = 1;
+    }
   }
-  if (t == 0 && (int64_t)nf + carry > a.total_pages) s_fail = 1;
   __syncthreads();
   if (s_fail) {
     if (t == 0) {
@@ -117,74 +178,86 @@ __global__ __launch_bounds__(kThreads) void admit_plan_kernel(AdmitArgs a) {
     }
     return;
   }
-  for (int h = t; h < a.H; h += kThreads) {
-    const int n = s_n[h];
-    if (n == 0) continue;
-    const int first = (int)(a.head_row[h] / a.page);
+  const int nf = s_nf;
+  for (int h = wid; h < a.H; h += kPlanWaves) {
+    const int n = s_n[h], first = nf + s_pg[h];
+    if (lane == 0) {
+      a.head_row[h] = (int64_t)first * a.page;
+      if (n > 0) a.global_lengths[a.layer * a.H + h] = n;
+    }
     const int pages = (n + a.page - 1) / a.page;
     int32_t* row = a.block_table + ((int64_t)a.layer * a.H + h) * a.max_pages + lb;
-    for (int i = 0; i < pages; ++i) row[i] = first + i;
-    a.global_lengths[a.layer * a.H + h] = n;
+    for (int i = lane; i < pages; i += 64) row[i] = first + i;
   }
   if (t == 0) {
-    *a.next_free = nf + carry;
+    *a.next_free = nf + s_total;
     *a.abort_flag = 0;
   }
 }
 
 // Stable compaction of admitted positions of [0, S-W) into the head's pages,
-// and the ring write of the last min(S, W) positions.
+// and the ring write of the last min(S, W) positions.  A workgroup takes 64
+// positions of one head: lane i of every wave holds flag i, so a ballot ranks
+// the rows, and the admitted positions between the count tile's start and
+// these are counted by the workgroup itself (at most 124 vector loads).  The
+// ring's W rows are then copied by W/64 workgroups per head.  Bound by
+// latency: with 2048 positions per workgroup and one load per thread in
+// flight a single workgroup copied a head's whole ring, and the admission of
+// 9001 tokens (8 heads, 20 % admitted, W 1024) took 73 us (count 4.6, plan
+// 5.4, scatter 63.8); it takes 12 us in this form.
 __global__ __launch_bounds__(kThreads) void admit_scatter_kernel(AdmitArgs a) {
-  __shared__ int s_tmp[kThreads];
-  __shared__ int s_src[kTile];
-  __shared__ int64_t s_dst[kTile];
-  __shared__ int s_n;
-  if (*a.abort_flag) return;
-  const int h = blockIdx.y, tile = blockIdx.x;
-  const int t = threadIdx.x;
+  __shared__ int s_src[kRows];
+  __shared__ int s_w[kThreads / 64];
+  const int h = blockIdx.y;
+  const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+  const int p0 = blockIdx.x * kRows;
   const int n_early = max(0, a.S - a.W);
   const int n_loc = min(a.S, a.W);
   const uint8_t* m = a.mask + (int64_t)h * a.m_sh;
-  const int p0 = tile * kTile + t * (kTile / kThreads);
-  // global part: positions p0 .. p0+7 of this thread, in order
-  int cnt = 0;
-  for (int k = 0; k < kTile / kThreads; ++k) {
-    const int p = p0 + k;
-    cnt += (p < n_early && m[p]) ? 1 : 0;
-  }
-  int total = 0;
-  int o = block_exclusive_scan_256(cnt, s_tmp, &total);
-  const int64_t base_row = a.head_row[h] + a.tile_base[h * a.ntiles + tile];
-  for (int k = 0; k < kTile / kThreads; ++k) {
-    const int p = p0 + k;
-    if (p < n_early && m[p]) {
-      s_src[o] = p;
-      s_dst[o] = base_row + o;
-      ++o;
-    }
-  }
+  const int p = p0 + lane;
+  const bool flag = p < a.S && m[p] != 0;
+  const int tile = p0 / kTile;
+  const int64_t row0 = a.head_row[h] + a.tile_base[h * a.ntiles + tile];
+  const int before = p0 < n_early ? wave_sum_int(count_flags(m, tile * kTile, p0, t, kThreads)) : 0;
+  if (*a.abort_flag) return;
+  const uint64_t adm = __builtin_amdgcn_ballot_w64(flag && p < n_early);
+  if (lane == 0) s_w[wid] = before;
+  if (wid == 0 && (adm >> lane & 1)) s_src[__builtin_popcountll(adm & ((1ull << lane) - 1))] = p;
   __syncthreads();
-  copy_rows(a.key + (int64_t)h * a.kv_sh, a.kv_ss, s_src, s_dst, total, a.D, a.pool_k);
-  copy_rows(a.value + (int64_t)h * a.kv_sh, a.kv_ss, s_src, s_dst, total, a.D, a.pool_v);
-  __syncthreads();
+  const int64_t base_row = row0 + ((s_w[0] + s_w[1]) + (s_w[2] + s_w[3]));
+  const uint16_t* key = a.key + (int64_t)h * a.kv_sh;
+  const uint16_t* value = a.value + (int64_t)h * a.kv_sh;
+  copy_rows2(key, value, a.kv_ss, __builtin_popcountll(adm), a.D, [&](unsigned r) { return s_src[r]; },
+             [&](unsigned r) { return base_row + r; }, a.pool_k, a.pool_v);
   // ring part: slot i <- position S - n_loc + i (src/modeling_layers.py:1290-1300)
   const int ring0 = a.S - n_loc;
-  const int lo = max(ring0, tile * kTile), hi = min(a.S, (tile + 1) * kTile);
-  if (t == 0) s_n = max(0, hi - lo);
-  const int64_t local_base = ((int64_t)a.layer * a.H + h) * a.W;
-  for (int p = lo + t; p < hi; p += kThreads) {
-    const int slot = p - ring0;
-    s_src[p - lo] = p;
-    s_dst[p - lo] = local_base + slot;
-    a.local_is_global[local_base + slot] = m[p] ? 1 : 0;
-  }
-  __syncthreads();
-  const int nr = s_n;
-  copy_rows(a.key + (int64_t)h * a.kv_sh, a.kv_ss, s_src, s_dst, nr, a.D, a.pool_k);
-  copy_rows(a.value + (int64_t)h * a.kv_sh, a.kv_ss, s_src, s_dst, nr, a.D, a.pool_v);
+  const int lo = max(ring0, p0), hi = min(a.S, p0 + kRows);
+  if (lo >= hi) return;
+  const int64_t slot0 = ((int64_t)a.layer * a.H + h) * a.W + (lo - ring0);
+  if (wid == 0 && p >= lo && p < hi) a.local_is_global[slot0 + (p - lo)] = flag ? 1 : 0;
+  copy_rows2(key, value, a.kv_ss, hi - lo, a.D, [&](unsigned r) { return lo + (int)r; },
+             [&](unsigned r) { return slot0 + r; }, a.pool_k, a.pool_v);
   if (a.pre_key && a.local_pre_key) {
     // local_pre_key is (L, H, W, D): its row index equals the pool's ring row
-    copy_rows(a.pre_key + (int64_t)h * a.pk_sh, a.pk_ss, s_src, s_dst, nr, a.D, a.local_pre_key);
+    const unsigned chunks = a.D / 8, total = (hi - lo) * chunks;
+    const uint16_t* pk = a.pre_key + (int64_t)h * a.pk_sh;
+    constexpr int U = 4;
+    for (unsigned e0 = t; e0 < total; e0 += kThreads * U) {
+      u32x4_t v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const unsigned e = min(e0 + u * kThreads, total - 1);
+        const unsigned r = e / chunks;
+        v[u] = *(const u32x4_t*)(pk + (int64_t)(lo + (int)r) * a.pk_ss + (e - r * chunks) * 8);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const unsigned e = e0 + u * kThreads;
+        if (e >= total) break;
+        const unsigned r = e / chunks;
+        *(u32x4_t*)(a.local_pre_key + (slot0 + r) * a.D + (e - r * chunks) * 8) = v[u];
+      }
+    }
   }
 }
 
@@ -432,10 +505,13 @@ extern "C" int wgkv_prefill_admit(
   ws += (size_t)num_kv_heads * a.ntiles * sizeof(int32_t);
   a.abort_flag = (int32_t*)ws;
   hipStream_t st = (hipStream_t)stream;
-  dim3 grid(a.ntiles, num_kv_heads);
-  hipLaunchKernelGGL(admit_count_kernel, grid, dim3(kThreads), 0, st, a);
-  hipLaunchKernelGGL(admit_plan_kernel, dim3(1), dim3(kThreads), 0, st, a);
-  hipLaunchKernelGGL(admit_scatter_kernel, grid, dim3(kThreads), 0, st, a);
+  if ((int64_t)a.ntiles * num_kv_heads <= kPlanCounts) {
+    hipLaunchKernelGGL(admit_plan_kernel<true>, dim3(1), dim3(kPlanThreads), 0, st, a);
+  } else {
+    hipLaunchKernelGGL(admit_count_kernel, dim3(a.ntiles, num_kv_heads), dim3(kThreads), 0, st, a);
+    hipLaunchKernelGGL(admit_plan_kernel<false>, dim3(1), dim3(kPlanThreads), 0, st, a);
+  }
+  hipLaunchKernelGGL(admit_scatter_kernel, dim3((seq_len + kRows - 1) / kRows, num_kv_heads), dim3(kThreads), 0, st, a);
   return hipGetLastError() == hipSuccess ? WGKV_OK : WGKV_ERR_HIP;
 }
 

@@ -127,6 +127,28 @@ WGKV_DEVICE int block_exclusive_scan_256(int v, int* s_tmp /* >= 4 ints */, int*
   return before + incl - v;
 }
 
+// This thread's share (t of n threads, n >= 16) of the nonzero flags in
+// m[lo, hi): whole 16-byte groups as vectors, the ends -- rows of odd length
+// start anywhere -- as bytes.
+WGKV_DEVICE int count_flags(const uint8_t* m, int lo, int hi, int t, int n) {
+  if (hi <= lo) return 0;
+  const uint8_t* p = m + lo;
+  const int head = min((int)((16 - ((uintptr_t)p & 15)) & 15), hi - lo);
+  const int groups = (hi - lo - head) >> 4;
+  const int tail = hi - lo - head - groups * 16;
+  int c = 0;
+  if (t < head) c += p[t] != 0;
+  if (t < tail) c += m[hi - tail + t] != 0;
+  const u32x4_t* v = (const u32x4_t*)(p + head);
+  for (int g = t; g < groups; g += n) {
+    const u32x4_t w = v[g];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)  // bit 7 of each nonzero byte
+      c += __builtin_popcount((((w[i] & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w[i]) & 0x80808080u);
+  }
+  return c;
+}
+
 #define WGKV_HIP_CHECK(expr)                       \
   do {                                             \
     hipError_t _e = (expr);                        \
