@@ -54,3 +54,25 @@ def test_long_prompts(S, W):
     rng = np.random.default_rng(S)
     m = rng.random((1, 8, S)) < 0.2
     check(m, W)
+
+
+@pytest.mark.parametrize("S", [1023, 1024, 1025, 1088, 1089, 2049, 2112, 2113, 196608, 196672, 196673])
+def test_tile_edges_and_unaligned_rows(S):
+    """Edges of the kernel's tiles (1024 positions, 4096 past 196608 listed
+    ones), with mask rows that start at any byte and nonzero flags other than
+    1: whole numbers, bit for bit."""
+    import wgkv
+    H, W = 3, 128
+    rng = np.random.default_rng(S)
+    flags = (rng.random((1, H, S + 3)) < 0.3).astype(np.uint8) * rng.integers(1, 256, (1, H, S + 3)).astype(np.uint8)
+    buf = np.zeros(flags.size + 1, dtype=np.uint8)
+    buf[1:] = flags.ravel()
+    mask = torch.from_numpy(buf).cuda()[1:].view(1, H, S + 3)[:, :, :S]
+    got = [t.cpu().numpy() for t in wgkv.generate_sparse_indices(mask, W, 1, H, S, exact_width=True)]
+    ref = meta.generate_sparse_indices(flags[:, :, :S] != 0, W, 64)
+    for g, r in zip(got[:3], ref[:3]):
+        assert np.array_equal(g, r)
+    assert got[3].shape == ref[3].shape
+    for h in range(H):
+        n = int(ref[2][0, h].max(initial=0))
+        assert np.array_equal(got[3][0, h, 0, :n], ref[3][0, h, 0, :n])

@@ -6,16 +6,28 @@
 //
 // Count blocks: block 0 is position 0 alone, block k >= 1 covers
 // [1 + (k-1)*bs, 1 + k*bs) -- the grouping whose running sums give, for row
-// block r >= P, the number of admitted positions below r*bs - W + 1.
-// One workgroup per (b, h) walks the count blocks in tiles of 256 with a
-// block-wide scan, writes column_count and compacts the admitted positions of
-// the listed range (positions < 1 + bs*((S-1)/bs)) in ascending order.  One
-// extra workgroup writes the band tables, which depend only on (W, S, bs).
+// block r >= P, the number of admitted positions below r*bs - W + 1.  Block k
+// thus ends at position k*bs, and column_count[k + P] is the inclusive count
+// there; the listed range is [0, (R-1)*bs].
+//
+// A workgroup takes `tile` consecutive positions of one (b, h).  It counts
+// the flags before its tile itself (16 per load, an L2 read after the first
+// tile), so no workgroup waits for another and one launch does it all; then
+// thread t takes positions t, t + 256, ... of the tile, a ballot ranks a wave's
+// 64 flags and one scan over the tile's (step, wave) counts places them.  The
+// reads before the tile grow with the square of the prompt, so long prompts
+// take larger tiles.  Bound by latency (a few memory round trips): one
+// workgroup per head walking 64-flag blocks byte by byte took 22 us at 9001
+// tokens and 17 us at 777 (8 heads); this takes 4.3 and 3.8 us.  The workgroups
+// after the last head's write the band tables, which depend only on
+// (W, S, bs).
 #include "wgkv_common.h"
 
 namespace {
 
 constexpr int kThreads = 256;
+constexpr int kWaves = kThreads / 64;
+constexpr int kShortList = 196608;  // listed positions up to this take 1024-position tiles
 
 struct MetaArgs {
   const uint8_t* mask;
@@ -27,63 +39,71 @@ struct MetaArgs {
   int32_t* column_index;
   int col_cap;
   int32_t* column_total;
+  int tiles;  // per (b, h)
 };
 
+template <int STEPS>  // 256-position steps per tile
 __global__ __launch_bounds__(kThreads) void prefill_meta_kernel(MetaArgs a) {
-  __shared__ int s_tmp[kThreads];
-  const int t = threadIdx.x;
-  const int BH = a.B * a.H;
-  if ((int)blockIdx.x == BH) {
+  __shared__ int s_pre[kWaves];
+  __shared__ int s_cnt[STEPS * kWaves];
+  const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+  const int bh = blockIdx.x / a.tiles, tile = blockIdx.x - bh * a.tiles;
+  if (bh == a.B * a.H) {
     // band tables (one row per row block, P+1 entries each)
     const int width = a.P + 1;
     const int last_first = max(0, (a.R - 1) * a.bs - a.W + 1);
     const int last_count = (a.S - last_first + a.bs - 1) / a.bs;
-    for (int r = t; r < a.R; r += kThreads) {
-      int cnt;
-      if (r < a.P) {
-        cnt = r + 1;
-        for (int c = 0; c < width; ++c) a.block_offset[r * width + c] = c < a.P ? c * a.bs : 0;
-      } else {
-        cnt = a.P + 1;
-        for (int c = 0; c < width; ++c) a.block_offset[r * width + c] = 1 + (r - a.P + c) * a.bs;
-      }
-      a.block_count[r] = r == a.R - 1 ? last_count : cnt;
+    const int stride = a.tiles * kThreads;
+    for (int64_t e = (int64_t)tile * kThreads + t; e < (int64_t)a.R * width; e += stride) {
+      const int r = (int)(e / width), c = (int)(e - (int64_t)r * width);
+      a.block_offset[e] = r < a.P ? (c < a.P ? c * a.bs : 0) : 1 + (r - a.P + c) * a.bs;
+      if (c == 0) a.block_count[r] = r == a.R - 1 ? last_count : r < a.P ? r + 1 : width;
     }
     return;
   }
-  const int bh = blockIdx.x;
   const int b = bh / a.H, h = bh - b * a.H;
   const uint8_t* m = a.mask + (int64_t)b * a.m_sb + (int64_t)h * a.m_sh;
   int32_t* cc = a.column_count + (int64_t)bh * a.R;
   int32_t* ci = a.column_index + (int64_t)bh * a.col_cap;
-  for (int r = t; r < min(a.P, a.R); r += kThreads) cc[r] = 0;
+  const int n_list = (a.R - 1) * a.bs + 1;
+  const int p0 = tile * (STEPS * kThreads);
+  if (tile == 0)
+    for (int r = t; r < min(a.P, a.R); r += kThreads) cc[r] = 0;
 
-  const int nblk = a.R;  // count blocks 0 .. (S-1)/bs
-  int carry = 0;
-  for (int base = 0; base < nblk; base += kThreads) {
-    const int k = base + t;
-    int lo = 0, hi = 0;
-    if (k < nblk) {
-      lo = k == 0 ? 0 : 1 + (k - 1) * a.bs;
-      hi = k == 0 ? 1 : min(a.S, 1 + k * a.bs);
-    }
-    int cnt = 0;
-    for (int p = lo; p < hi; ++p) cnt += m[p] != 0;
-    int total = 0;
-    const int excl = block_exclusive_scan_256(cnt, s_tmp, &total);
-    if (k < nblk) {
-      const int incl = carry + excl + cnt;
-      if (k + a.P < a.R) cc[k + a.P] = incl;
-      int o = carry + excl;
-      for (int p = lo; p < hi; ++p)
-        if (m[p]) {
-          if (o < a.col_cap) ci[o] = p;
-          ++o;
-        }
-    }
-    carry += total;
+  // this tile's flags and the count before it
+  uint64_t bal[STEPS];
+#pragma unroll
+  for (int i = 0; i < STEPS; ++i) {
+    const int p = p0 + i * kThreads + t;
+    bal[i] = __builtin_amdgcn_ballot_w64(p < n_list && m[p] != 0);
   }
-  if (t == 0 && a.column_total) a.column_total[bh] = carry;
+  const int pre = wave_sum_int(count_flags(m, 0, min(p0, n_list), t, kThreads));
+  if (lane == 0) {
+    s_pre[wid] = pre;
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i) s_cnt[i * kWaves + wid] = __builtin_popcountll(bal[i]);
+  }
+  __syncthreads();
+  int run = (s_pre[0] + s_pre[1]) + (s_pre[2] + s_pre[3]);  // admitted before this wave's 64 flags of the step
+#pragma unroll
+  for (int i = 0; i < STEPS; ++i) {
+    int mine = run;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      const int c = s_cnt[i * kWaves + w];
+      mine += w < wid ? c : 0;
+      run += c;
+    }
+    const int p = p0 + i * kThreads + t;
+    const bool f = bal[i] >> lane & 1;
+    const int rank = mine + __builtin_popcountll(bal[i] & ((1ull << lane) - 1));
+    if (f && rank < a.col_cap) ci[rank] = p;
+    if (p < n_list && p % a.bs == 0) {
+      const int r = p / a.bs + a.P;
+      if (r < a.R) cc[r] = rank + (f ? 1 : 0);
+    }
+  }
+  if (t == 0 && a.column_total && p0 < n_list && p0 + STEPS * kThreads >= n_list) a.column_total[bh] = run;
 }
 
 }  // namespace
@@ -115,7 +135,17 @@ extern "C" int wgkv_build_prefill_meta(
   a.column_index = column_index;
   a.col_cap = col_cap;
   a.column_total = column_total;
-  hipLaunchKernelGGL(prefill_meta_kernel, dim3(batch * num_kv_heads + 1), dim3(kThreads), 0,
-                     (hipStream_t)stream, a);
+  // Positions per workgroup: 1024 while the flags before a tile are read by few
+  // loads per thread, 4096 where those reads outweigh the tile's own work.  8
+  // heads, 1024 / 4096: 65536 positions 6.6 / 10.1 us, 131072 9.9 / 12.9,
+  // 262144 25.7 / 18.6, 400000 37.9 / 24.8.
+  const int n_list = (a.R - 1) * block + 1;
+  const int tile = n_list <= kShortList ? 1024 : 4096;
+  a.tiles = (n_list + tile - 1) / tile;
+  const dim3 grid((unsigned)a.tiles * (batch * num_kv_heads + 1));
+  if (tile == 1024)
+    hipLaunchKernelGGL(prefill_meta_kernel<4>, grid, dim3(kThreads), 0, (hipStream_t)stream, a);
+  else
+    hipLaunchKernelGGL(prefill_meta_kernel<16>, grid, dim3(kThreads), 0, (hipStream_t)stream, a);
   return hipGetLastError() == hipSuccess ? WGKV_OK : WGKV_ERR_HIP;
 }
