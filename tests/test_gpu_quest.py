@@ -209,3 +209,51 @@ def test_selection_matches_reference_golden(name):
             rows.append(sel_bt[0, h, :count].cpu().tolist())
         check_selection_against_golden(z, name, i, sc, st, sel_len[0].cpu().tolist(), rows)
     print(f"[quest golden] {name}: {len(sc['steps'])} steps, lengths exact, selections equal up to ties", flush=True)
+
+
+@pytest.mark.parametrize("scores_bf16", [False, True])
+@pytest.mark.parametrize("G,D", [(1, 128), (3, 64), (4, 128), (5, 8), (8, 256)])
+@pytest.mark.parametrize("budget", [64, 64 + 16, 64 + 16 * 40, 64 + 16 * 1500])
+def test_selection_exact_over_head_lengths(G, D, budget, scores_bf16):
+    """Heads from no page to more than the selection keeps in registers (8192
+    pages).  Queries and bounds are small integers, so every score is exact in
+    fp32 and ties are many: the selection must be the largest scores, equal
+    ones by page order, whole numbers bit for bit."""
+    import types
+    from wgkv import ops
+    W, P = 64, 16
+    fulls = [0, 1, 15, 16, 17, 63, 64, 65, 1023, 1024, 1025, 2049, 8192, 8193, 12000]
+    lens = [f * P + (i % 3) * 5 for i, f in enumerate(fulls)]
+    H, lb = len(fulls), W // P
+    g = torch.Generator().manual_seed(G * D + budget)
+    pages = [(n + P - 1) // P for n in lens]
+    total, width = H * lb + sum(pages), lb + max(pages)
+    perm = torch.randperm(total, generator=g).to(torch.int32)
+    table = torch.full((1, H, width), total - 1, dtype=torch.int32)
+    at = 0
+    for h, p in enumerate(pages):
+        table[0, h, :lb + p] = perm[at:at + lb + p]
+        at += lb + p
+    lo = torch.randint(-4, 3, (total, D), generator=g).float()
+    hi = lo + torch.randint(0, 3, (total, D), generator=g)
+    q = torch.randint(-2, 3, (H * G, D), generator=g).float()
+    bf = torch.bfloat16
+    c = types.SimpleNamespace(num_layers=1, num_kv_heads=H, head_dim=D, block_size=P, local_window_size=W,
+                              block_table=table.to(DEV), global_lengths=torch.tensor([lens], dtype=torch.int32).to(DEV),
+                              quest_block_key_min=lo.to(bf).to(DEV), quest_block_key_max=hi.to(bf).to(DEV))
+    print(f"[quest] exact G{G} D{D} budget{budget} bf16={scores_bf16}", flush=True)
+    sel_len, sel_bt = ops.quest_select(c, 0, q.to(bf).to(DEV), W, budget, scores_bf16=scores_bf16)
+    cap = (budget - W + P - 1) // P
+    for h in range(H):
+        full, rem = divmod(lens[h], P)
+        have = min(cap, pages[h])
+        keep = max(0, min(full, have - (1 if rem else 0)))
+        ids = table[0, h, lb:lb + full].long()
+        qq = q[h * G:(h + 1) * G, None]
+        s = (qq * torch.where(qq >= 0, hi[ids][None], lo[ids][None])).sum(-1)
+        s = (s.to(bf).float() if scores_bf16 else s).amax(0)
+        order = torch.sort(s, descending=True, stable=True).indices[:keep].sort().values
+        want = torch.cat((table[0, h, :lb], table[0, h, lb:][order],
+                          table[0, h, lb + full:lb + full + (1 if have > 0 and rem else 0)]))
+        assert int(sel_len[0, h]) == W + keep * P + (rem if have > 0 and rem else 0), h
+        assert torch.equal(sel_bt[0, h, :want.numel()].cpu(), want), h

@@ -12,10 +12,10 @@
 //     pages [from/page, ceil(len/page)) from the pool (the min / max over the
 //     page's valid rows, which equals the reference's incremental updates);
 //   * quest_scores_kernel: the page scores of every head into the workspace;
-//   * quest_select_kernel: one workgroup per head -- a 4-pass radix select
-//     of the k-th largest score, then a
-//     stable compaction that writes local pages, the kept full pages in page
-//     order and the partial page, and the head's token count.
+//   * quest_select_kernel: one workgroup per head -- the k-th largest score
+//     by bisection of its bits, then a stable compaction that writes local
+//     pages, the kept full pages in page order and the partial page, and the
+//     head's token count.
 // Scores are fp32, or (scores_bf16) rounded as the reference's bf16 torch ops
 // round them: each product q_d * bound_d to bf16, the fp32 sum over d to
 // bf16.  Equal scores at the cut keep the lowest page index (the reference's
@@ -73,149 +73,242 @@ struct SelectArgs {
   const int32_t* len;  // global_lengths + layer * H
   const uint16_t* kmin;
   const uint16_t* kmax;
-  int H, G, D, page, local_tokens, budget, scores_bf16;
+  int H, G, D, page, local_tokens, scores_bf16;
+  int local_blocks, budget_blocks;  // pages of the local tokens and of the budget past them
   int32_t* sel_bt;     // (H, sel_cap)
   int sel_cap;
   int32_t* sel_len;    // (H)
   float* scores;       // workspace (H, max_pages)
 };
 
-// Page scores, grid (64, H): 16 lanes per page (8 d-values each, 16-byte
-// loads of the bounds), the lane partials summed with a 16-lane row
-// reduction; workgroups stride over the head's full pages.
+// Page scores: 16 lanes per page, 8 d-values each (16-byte loads of the
+// bounds; the queries' 8 values per group member held in registers), summed
+// per lane in d order and then over the 16 lanes; workgroups stride over the
+// head's full pages, two of them per lane group in flight.  Bound by latency
+// (a 128K prompt's 13.1K pages are 6.7 MB of bounds): the group size is a
+// template argument, as a runtime bound put the per-member sums in scratch
+// memory and read the queries from LDS value by value (30 us; now 6.2 us).
+template <int G, bool BF16>
 __global__ __launch_bounds__(kThreads) void quest_scores_kernel(SelectArgs a) {
-  __shared__ float s_q[8][256];
+  __shared__ __attribute__((aligned(16))) uint16_t s_q[G][256];
   const int h = blockIdx.y, t = threadIdx.x;
   const int full = a.len[h] / a.page;
-  for (int e = t; e < a.G * a.D; e += kThreads) {
+  if ((int)blockIdx.x * 16 >= full) return;
+  for (int e = t; e < G * a.D; e += kThreads) {
     const int g = e / a.D, d = e - g * a.D;
-    s_q[g][d] = bf(a.q[(int64_t)(h * a.G + g) * a.q_sh + d]);
+    s_q[g][d] = a.q[(int64_t)(h * G + g) * a.q_sh + d];
   }
   __syncthreads();
   const int32_t* bt = a.bt + (int64_t)h * a.max_pages + a.lb;
   float* sc = a.scores + (int64_t)h * a.max_pages;
   const int lane16 = t & 15, slot = t >> 4;  // 16 pages per pass
   const int nch = a.D / 8;                   // 8-value chunks per row (<= 32)
-  for (int p0 = blockIdx.x * 16; p0 < full; p0 += gridDim.x * 16) {
-    const int p = p0 + slot;
-    const bool ok = p < full;
-    const int64_t pg = ok ? bt[p] : 0;
-    float s[8];
+  constexpr int U = 2;                       // passes in flight
+  const int step = gridDim.x * 16;
+  for (int p0 = blockIdx.x * 16 + slot; p0 < full + slot; p0 += step * U) {
+    int64_t row[U];
+    bool ok[U];
 #pragma unroll
-    for (int g = 0; g < 8; ++g) s[g] = 0.f;
+    for (int u = 0; u < U; ++u) {
+      ok[u] = p0 + u * step < full;
+      row[u] = (int64_t)bt[ok[u] ? p0 + u * step : 0] * a.D;
+    }
+    float s[U][G] = {};
     for (int c = lane16; c < nch; c += 16) {
-      const u32x4_t lo = ok ? *(const u32x4_t*)(a.kmin + pg * a.D + c * 8) : (u32x4_t){0u, 0u, 0u, 0u};
-      const u32x4_t hi = ok ? *(const u32x4_t*)(a.kmax + pg * a.D + c * 8) : (u32x4_t){0u, 0u, 0u, 0u};
+      u32x4_t lo[U], hi[U];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float l = (e & 1) ? bf16hi(lo[e >> 1]) : bf16lo(lo[e >> 1]);
-        const float u = (e & 1) ? bf16hi(hi[e >> 1]) : bf16lo(hi[e >> 1]);
-        for (int g = 0; g < a.G; ++g) {
-          const float qd = s_q[g][c * 8 + e];
-          const float b = qd >= 0.f ? u : l;
-          // a product of two bf16 values is exact in fp32; bf16 ops round it
-          s[g] = a.scores_bf16 ? s[g] + round_bf16f(qd * b) : fmaf(qd, b, s[g]);
+      for (int u = 0; u < U; ++u) {
+        lo[u] = *(const u32x4_t*)(a.kmin + row[u] + c * 8);
+        hi[u] = *(const u32x4_t*)(a.kmax + row[u] + c * 8);
+      }
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        const u32x4_t qv = *(const u32x4_t*)&s_q[g][c * 8];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float q0 = bf16lo(qv[e]), q1 = bf16hi(qv[e]);
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const float b0 = q0 >= 0.f ? bf16lo(hi[u][e]) : bf16lo(lo[u][e]);
+            const float b1 = q1 >= 0.f ? bf16hi(hi[u][e]) : bf16hi(lo[u][e]);
+            // a product of two bf16 values is exact in fp32; bf16 ops round it
+            if (BF16) {
+              const uint32_t r = pack_bf16x2(q0 * b0, q1 * b1);
+              s[u][g] = (s[u][g] + bf16lo(r)) + bf16hi(r);
+            } else {
+              s[u][g] = fmaf(q1, b1, fmaf(q0, b0, s[u][g]));
+            }
+          }
         }
       }
     }
-    float best = -INFINITY;
-    for (int g = 0; g < a.G; ++g) {
-      const float v = row_sum16(s[g]);
-      best = fmaxf(best, a.scores_bf16 ? round_bf16f(v) : v);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      float best = -INFINITY;
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        const float v = row_sum16(s[u][g]);
+        best = fmaxf(best, BF16 ? round_bf16f(v) : v);
+      }
+      if (ok[u] && lane16 == 0) sc[p0 + u * step] = best;
     }
-    if (ok && lane16 == 0) sc[p] = best;
   }
 }
 
 // order-preserving map of an fp32 to uint32 (larger float -> larger key)
 __device__ __forceinline__ uint32_t fkey(float f) {
   const uint32_t u = __float_as_uint(f);
-  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+  return u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);
 }
 
-__global__ __launch_bounds__(kThreads) void quest_select_kernel(SelectArgs a) {
-  __shared__ int s_hist[256];
-  __shared__ int s_tmp[kThreads];
-  __shared__ uint32_t s_prefix;
-  __shared__ int s_need;
-  const int h = blockIdx.x, t = threadIdx.x;
-  const int n = a.len[h];
-  const int full = n / a.page, rem = n % a.page;
-  const int local_blocks = (a.local_tokens + a.page - 1) / a.page;
-  const int budget_blocks = (max(a.budget - a.local_tokens, 0) + a.page - 1) / a.page;
-  const int gblocks = (n + a.page - 1) / a.page;
-  const int capacity = min(budget_blocks, gblocks);
-  const bool partial = capacity > 0 && rem > 0;
-  const int k = capacity - (rem > 0 ? 1 : 0);  // full pages to keep
-  const int32_t* bt = a.bt + (int64_t)h * a.max_pages;
-  int32_t* out = a.sel_bt + (int64_t)h * a.sel_cap;
-  float* sc = a.scores + (int64_t)h * a.max_pages;
+// The selection of a head's `keep` largest of `full` page scores (0 < keep <
+// full) by one workgroup, kept pages written in page order from out on.  The
+// keep-th largest key T is found two bits at a time -- the largest T with at
+// least `keep` keys >= T -- with counts from ballots: no histogram, whose
+// bins the equal exponents of page scores crowd into.  Scores rounded to bf16
+// differ only in the key's upper half: 8 steps instead of 16.  With STAGED
+// the keys are read once and kept in LDS (heads of up to kMaxKeys pages),
+// else the scores are read again in every step.
+constexpr int kMaxKeys = 12288;  // a multiple of 8 * kThreads
+constexpr int kWaves = kThreads / 64;
+constexpr int kRowGroup = 64;  // rows of kThreads pages placed per scan
 
-  for (int i = t; i < local_blocks; i += kThreads) out[i] = bt[i];
-  const bool all = k >= full;
-  const int keep = k <= 0 ? 0 : (all ? full : k);
-
-  if (keep > 0 && !all) {
-    // radix select of the key of the keep-th largest score
-    if (t == 0) {
-      s_prefix = 0;
-      s_need = keep;
+template <bool BF16, bool STAGED>
+__device__ void select_pages(const float* sc, int full, int keep, const int32_t* pages, int32_t* out,
+                             uint32_t* s_key, int (*s_cnt)[3][kWaves], int* s_pref, int* s_tmp) {
+  constexpr int BITS = BF16 ? 16 : 32;
+  const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+  const int rows = (full + kThreads - 1) / kThreads;  // of kThreads pages
+  // key of page p, 0 past the head's pages: below every tested value
+  auto read_key = [&](int p) {
+    const uint32_t x = fkey(sc[min(p, full - 1)]) >> (32 - BITS);
+    return p < full ? x : 0u;
+  };
+  auto key_at = [&](int p) { return STAGED ? s_key[p] : read_key(p); };
+  if (STAGED) {  // whole groups of eight rows; each thread reads back only its own keys: no barrier
+    for (int r0 = 0; r0 < rows; r0 += 8) {
+      uint32_t x[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = read_key((r0 + j) * kThreads + t);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s_key[(r0 + j) * kThreads + t] = x[j];
+    }
+  }
+  uint32_t T = 0;
+  int above = 0;  // keys >= T's last tested successor: keys > T at the end
+#pragma unroll 1
+  for (int shift = BITS - 2, step = 0; shift >= 0; shift -= 2, step ^= 1) {
+    int c[3] = {0, 0, 0};
+#pragma unroll 1
+    for (int r0 = 0; r0 < rows; r0 += 8) {
+      uint32_t x[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = key_at((r0 + j) * kThreads + t);
+#pragma unroll
+      for (int d = 0; d < 3; ++d)
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          c[d] += __builtin_popcountll(__builtin_amdgcn_ballot_w64(x[j] >= (T | ((uint32_t)(d + 1) << shift))));
+    }
+    // a step's counts are read before the next step's barrier: two sets suffice
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+      if (lane == 0) s_cnt[step][d][wid] = c[d];
+    __syncthreads();
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+      c[d] = (s_cnt[step][d][0] + s_cnt[step][d][1]) + (s_cnt[step][d][2] + s_cnt[step][d][3]);
+    const int digit = c[2] >= keep ? 3 : c[1] >= keep ? 2 : c[0] >= keep ? 1 : 0;
+    T |= (uint32_t)digit << shift;
+    if (digit < 3) above = c[digit];
+  }
+  T = __builtin_amdgcn_readfirstlane(T);
+  // kept: key > T, plus the first need_eq pages (in page order) with key ==
+  // T.  kRowGroup rows at a time: each (row, wave)'s two counts packed in one
+  // word, their prefix in page order, then the kept pages' places.
+  const int need_eq = keep - above;
+  int base_gt = 0, base_eq = 0;  // before the group (a group's own counts fit 16 bits)
+  for (int g0 = 0; g0 < rows; g0 += kRowGroup) {
+    const int gr = min(kRowGroup, rows - g0);
+    __syncthreads();
+    for (int r = 0; r < gr; ++r) {
+      const int p = (g0 + r) * kThreads + t;
+      const uint32_t x = key_at(p);
+      const int gt = __builtin_popcountll(__builtin_amdgcn_ballot_w64(x > T));
+      const int eq = __builtin_popcountll(__builtin_amdgcn_ballot_w64(x == T && p < full));
+      if (lane == 0) s_pref[r * kWaves + wid] = gt << 16 | eq;
     }
     __syncthreads();
-    for (int shift = 24; shift >= 0; shift -= 8) {
-      s_hist[t] = 0;
-      __syncthreads();
-      const uint32_t hi_mask = shift == 24 ? 0u : (0xffffffffu << (shift + 8));
-      const uint32_t prefix = s_prefix;
-      for (int p = t; p < full; p += kThreads) {
-        const uint32_t key = fkey(sc[p]);
-        if ((key & hi_mask) == (prefix & hi_mask)) atomicAdd(&s_hist[(key >> shift) & 255], 1);
-      }
-      __syncthreads();
-      // counts from the top bin down: thread t holds bin 255 - t
-      const int c = s_hist[255 - t];
-      int total = 0;
-      const int above = block_exclusive_scan_256(c, s_tmp, &total);  // keys in higher bins
-      const int need = s_need;
-      __syncthreads();
-      if (above < need && need <= above + c) {  // the bin holding the need-th key
-        s_prefix = prefix | ((uint32_t)(255 - t) << shift);
-        s_need = need - above;
-      }
-      __syncthreads();
+    int total = 0;
+    const int pref = block_exclusive_scan_256(t < gr * kWaves ? s_pref[t] : 0, s_tmp, &total);
+    s_pref[t] = pref;
+    __syncthreads();
+    for (int r = 0; r < gr; ++r) {
+      const int p = (g0 + r) * kThreads + t;
+      const uint32_t x = key_at(p);
+      const uint64_t gt = __builtin_amdgcn_ballot_w64(x > T);
+      const uint64_t eq = __builtin_amdgcn_ballot_w64(x == T && p < full);
+      const int before = s_pref[r * kWaves + wid];
+      const uint64_t below = (1ull << lane) - 1;
+      const int rank_gt = base_gt + (before >> 16) + __builtin_popcountll(gt & below);
+      const int rank_eq = base_eq + (before & 0xffff) + __builtin_popcountll(eq & below);
+      if ((gt >> lane & 1) || ((eq >> lane & 1) && rank_eq < need_eq)) out[rank_gt + min(rank_eq, need_eq)] = pages[p];
     }
-    // kept: key > T, plus the first s_need pages (in page order) with key == T;
-    // thread t owns the contiguous pages [t*per, (t+1)*per)
-    const uint32_t T = s_prefix;
-    const int need_eq = s_need;
-    const int per = (full + kThreads - 1) / kThreads;
-    const int p0 = min(full, t * per), p1 = min(full, p0 + per);
-    int n_eq = 0;
-    for (int p = p0; p < p1; ++p) n_eq += fkey(sc[p]) == T ? 1 : 0;
-    int tot = 0;
-    int eq_rank = block_exclusive_scan_256(n_eq, s_tmp, &tot);
-    int n_take = 0;
-    {
-      int r = eq_rank;
-      for (int p = p0; p < p1; ++p) {
-        const uint32_t key = fkey(sc[p]);
-        if (key > T) ++n_take;
-        else if (key == T) n_take += (r++ < need_eq) ? 1 : 0;
-      }
-    }
-    int pos = local_blocks + block_exclusive_scan_256(n_take, s_tmp, &tot);
-    for (int p = p0; p < p1; ++p) {
-      const uint32_t key = fkey(sc[p]);
-      bool take = key > T;
-      if (key == T) take = eq_rank++ < need_eq;
-      if (take) out[pos++] = bt[a.lb + p];
-    }
+    base_gt += total >> 16;
+    base_eq += total & 0xffff;
+  }
+}
+
+// One workgroup per head.  Bound by latency (a few memory round trips and the
+// steps' barriers); four waves rather than sixteen, whose barriers and scalar
+// counting cost more than the keys.  1638 pages per head, 8 heads: 15.0 us
+// with four LDS-histogram passes over the scores in memory, 10.4 us in this
+// form.
+template <bool BF16>
+__global__ __launch_bounds__(kThreads) void quest_select_kernel(SelectArgs a) {
+  __shared__ uint32_t s_key[kMaxKeys];
+  __shared__ int s_cnt[2][3][kWaves];
+  __shared__ int s_pref[kRowGroup * kWaves];
+  __shared__ int s_tmp[kThreads];
+  const int h = blockIdx.x, t = threadIdx.x;
+  const int32_t* bt = a.bt + (int64_t)h * a.max_pages;
+  int32_t* out = a.sel_bt + (int64_t)h * a.sel_cap;
+  const float* sc = a.scores + (int64_t)h * a.max_pages;
+  const int n = a.len[h];
+  const int local_blocks = a.local_blocks;
+  for (int i = t; i < local_blocks; i += kThreads) out[i] = bt[i];
+  const int full = n / a.page, rem = n - full * a.page;
+  const int capacity = min(a.budget_blocks, full + (rem > 0 ? 1 : 0));
+  const bool partial = capacity > 0 && rem > 0;
+  const int k = capacity - (rem > 0 ? 1 : 0);  // full pages to keep
+  const bool all = k >= full;
+  const int keep = k <= 0 ? 0 : (all ? full : k);
+  if (keep > 0 && !all) {
+    if (full <= kMaxKeys)
+      select_pages<BF16, true>(sc, full, keep, bt + a.lb, out + local_blocks, s_key, s_cnt, s_pref, s_tmp);
+    else
+      select_pages<BF16, false>(sc, full, keep, bt + a.lb, out + local_blocks, s_key, s_cnt, s_pref, s_tmp);
   } else if (keep > 0) {
     for (int p = t; p < keep; p += kThreads) out[local_blocks + p] = bt[a.lb + p];
   }
   if (t == 0) {
     if (partial) out[local_blocks + keep] = bt[a.lb + full];
     a.sel_len[h] = a.local_tokens + keep * a.page + (partial ? rem : 0);
+  }
+}
+
+template <int G>
+void launch_select(const SelectArgs& a, hipStream_t st) {
+  // a head's pages over at least 64 workgroups, the call over about 1024; no
+  // more than its table could fill
+  const int most = (a.max_pages - a.lb + 15) / 16, want = max(64, 1024 / a.H);
+  const dim3 grid(max(1, min(most, want)), a.H);
+  if (a.scores_bf16) {
+    hipLaunchKernelGGL((quest_scores_kernel<G, true>), grid, dim3(kThreads), 0, st, a);
+    hipLaunchKernelGGL(quest_select_kernel<true>, dim3(a.H), dim3(kThreads), 0, st, a);
+  } else {
+    hipLaunchKernelGGL((quest_scores_kernel<G, false>), grid, dim3(kThreads), 0, st, a);
+    hipLaunchKernelGGL(quest_select_kernel<false>, dim3(a.H), dim3(kThreads), 0, st, a);
   }
 }
 
@@ -284,14 +377,23 @@ extern "C" int wgkv_quest_select(
   a.D = head_dim;
   a.page = page_size;
   a.local_tokens = local_tokens;
-  a.budget = token_budget;
+  a.local_blocks = local_blocks;
+  a.budget_blocks = budget_blocks;
   a.scores_bf16 = scores_bf16 ? 1 : 0;
   a.sel_bt = sel_block_table;
   a.sel_cap = sel_cap;
   a.sel_len = sel_seqlens;
   a.scores = (float*)workspace;
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(quest_scores_kernel, dim3(64, num_kv_heads), dim3(kThreads), 0, st, a);
-  hipLaunchKernelGGL(quest_select_kernel, dim3(num_kv_heads), dim3(kThreads), 0, st, a);
+  switch (G) {
+    case 1: launch_select<1>(a, st); break;
+    case 2: launch_select<2>(a, st); break;
+    case 3: launch_select<3>(a, st); break;
+    case 4: launch_select<4>(a, st); break;
+    case 5: launch_select<5>(a, st); break;
+    case 6: launch_select<6>(a, st); break;
+    case 7: launch_select<7>(a, st); break;
+    default: launch_select<8>(a, st); break;
+  }
   return hipGetLastError() == hipSuccess ? WGKV_OK : WGKV_ERR_HIP;
 }
