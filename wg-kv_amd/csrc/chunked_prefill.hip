@@ -20,8 +20,8 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
-constexpr int kTile = 512;   // virtual positions per scan tile
-constexpr int kBlk = 64;
+constexpr int kBlk = 64;      // virtual positions per scatter step
+constexpr int kMaxSpan = 8;   // steps per workgroup at most
 
 struct ChunkArgs {
   const uint16_t* key;
@@ -31,7 +31,6 @@ struct ChunkArgs {
   int64_t pk_sh, pk_ss;
   const uint8_t* mask;  // chunk flags (H, C)
   int64_t m_sh;
-  int mask_vec16;       // mask rows 16-byte aligned (16 flags per load)
   int layer, H, C, D, W, page, max_tokens_per_head, c0;
   int64_t total_pages;
   uint16_t* pool_k;
@@ -45,7 +44,7 @@ struct ChunkArgs {
   int32_t* status;
   int32_t* column_count;  // (H, R_chunk)
   int r0, rchunk;         // first global row block of the chunk, row blocks in the chunk
-  int ntiles;             // kTile-position tiles of the virtual sequence
+  int span;               // 64-position steps per admission workgroup
   // workspace, written by stage 0 and read by stage 1
   int32_t* adm;           // (H) positions admitted by the chunk
   int32_t* gl_before;     // (H) global lengths before the chunk
@@ -56,148 +55,88 @@ struct ChunkArgs {
 constexpr int kMaxHeads = 1024;
 
 // Virtual sequence of a chunk: ring positions (c0 > 0 only) then the chunk.
-__device__ __forceinline__ int vlen(const ChunkArgs& a) { return (a.c0 > 0 ? a.W : 0) + a.C; }
+__host__ __device__ __forceinline__ int vlen(const ChunkArgs& a) { return (a.c0 > 0 ? a.W : 0) + a.C; }
 __device__ __forceinline__ int vring(const ChunkArgs& a) { return a.c0 > 0 ? a.W : 0; }
 
-__device__ __forceinline__ bool vflag(const ChunkArgs& a, int h, int v) {
+// Admitted flags of head h among the first n virtual positions, this thread's
+// share (t of nt threads).
+__device__ __forceinline__ int vcount(const ChunkArgs& a, int h, int n, int t, int nt) {
   const int nr = vring(a);
-  if (v < nr) return a.local_is_global[((int64_t)a.layer * a.H + h) * a.W + v] != 0;
-  return a.mask[(int64_t)h * a.m_sh + (v - nr)] != 0;
+  int c = count_flags(a.mask + (int64_t)h * a.m_sh, 0, n - nr, t, nt);
+  if (nr > 0) c += count_flags(a.local_is_global + ((int64_t)a.layer * a.H + h) * a.W, 0, min(nr, n), t, nt);
+  return c;
 }
 
-// Admitted flags among virtual positions [v, min(v + 16, lim)) of head h
-// (flags are 0/1 bytes, so popcounts of the 16 bytes count them).  The ring
-// length W and v are multiples of 16, so the 16 positions lie all in the
-// ring or all in the chunk; reads never pass the chunk's own flags (v < lim
-// <= chunk_len + ring, and lim - v < 16 only at the admission range's end,
-// which lies W - 16 or more flags before the end of the chunk).
-__device__ __forceinline__ int count16(const ChunkArgs& a, int h, int v, int lim) {
-  const int nr = vring(a);
-  const int n = min(16, lim - v);
-  const uint8_t* p = v < nr ? a.local_is_global + ((int64_t)a.layer * a.H + h) * a.W + v
-                            : a.mask + (int64_t)h * a.m_sh + (v - nr);
-  u32x4_t w;
-  if (v < nr || a.mask_vec16) {
-    w = *(const u32x4_t*)p;
-  } else {
-    w = (u32x4_t){0u, 0u, 0u, 0u};
-    for (int i = 0; i < n; ++i) w[i >> 2] |= (uint32_t)p[i] << (8 * (i & 3));
-  }
-  if (n < 16) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int keep = min(4, max(0, n - 4 * q));  // bytes of word q inside the range
-      w[q] &= keep == 4 ? ~0u : ((1u << (8 * keep)) - 1u);
-    }
-  }
-  return __builtin_popcount(w[0]) + __builtin_popcount(w[1]) + __builtin_popcount(w[2]) + __builtin_popcount(w[3]);
-}
-
-// Admission of one chunk in one launch (workgroup = kTile virtual positions
-// of one head).  Every workgroup first counts the admitted flags of every
-// head and makes the same plan from them -- totals, capacity checks before
-// any write, pages bump-allocated in head order -- so no workgroup waits for
-// another; then it compacts its own tile into the head's pages (new pages are
-// numbered arithmetically from the plan, so the block-table entries written
-// here are not read back) and writes the column counts of the row blocks
-// whose band starts inside its tile: the count of row block r is the number
-// of admitted positions below p = 64 r - W + 1, i.e. the inclusive count at
-// virtual index p - 1 - base.  The global lengths and the bump pointer are
-// left to stage 1 (every workgroup here reads the lengths from before the
-// chunk).  Independent loads are issued together: the tile's flags, every
-// head's length and the 16-flag count loads, so the launch waits on memory
-// about three times (flags and lengths, existing page ids, K/V rows).
+// Admission of one chunk in one launch (workgroup = `span` steps of 64
+// virtual positions of one head).  Every workgroup first counts the admitted
+// flags of every head (a wave per head) and makes the same plan from them --
+// totals, capacity checks before any write, pages bump-allocated in head order
+// -- so no workgroup waits for another; then it compacts its own positions
+// into the head's pages (new pages are numbered arithmetically from the plan,
+// so the block-table entries written here are not read back) and writes the
+// column counts of the row blocks whose band starts inside them: the count of
+// row block r is the number of admitted positions below p = 64 r - W + 1,
+// i.e. the inclusive count at virtual index p - 1 - base, the first of a
+// step.  The global lengths and the bump pointer are left to stage 1 (every
+// workgroup here reads the lengths from before the chunk).
+//
+// Bound by latency: the launch waits on memory about three times (flags and
+// lengths, the head's last page id, K/V rows).  64 positions per workgroup
+// give 512 workgroups for a 4096-token chunk of 8 heads, each copying its
+// ~13 rows in one batch of loads; 512 positions and one copy in flight per
+// thread took 17.4 us, with the counts added into LDS by every thread; this
+// takes 9.5 us.  span grows with heads x positions (wgkv_chunk_cache_update).
 __global__ __launch_bounds__(kThreads) void chunk_admit_kernel(ChunkArgs a) {
-  constexpr int kPer = kTile / kThreads;
-  constexpr int kCnt = 16;       // flags per count load
-  constexpr int kLoads = 16;     // count loads per thread issued together
   __shared__ int s_tot[kMaxHeads];    // admitted positions of each head
-  __shared__ int s_first[kMaxHeads];  // first new page of each head, relative to the bump pointer
-  __shared__ int s_tmp[kThreads];
   __shared__ int s_wave[kWaves];
-  __shared__ int s_pre, s_fail, s_total_pages, s_nf;
-  __shared__ int s_src[kTile];        // virtual index
-  __shared__ int64_t s_dst[kTile];    // pool row
+  __shared__ int s_first, s_fail, s_total_pages;
+  __shared__ int s_src[kBlk];         // row of the step's source
+  __shared__ int64_t s_dst[kBlk];     // pool row
   const int h = blockIdx.y, tile = blockIdx.x;
   const int t = threadIdx.x;
   const int lane = t & 63, wid = t >> 6;
   const int nr = vring(a);
   const int n_adm = vlen(a) - a.W;  // admission range [0, n_adm) of the virtual sequence
   const int lb = a.W / a.page;
+  const int v0 = tile * a.span * kBlk;
+  const int32_t* lens = a.global_lengths + a.layer * a.H;
+  int32_t* bt = a.block_table + ((int64_t)a.layer * a.H + h) * a.max_pages + lb;
+  const uint8_t* ring_flags = a.local_is_global + ((int64_t)a.layer * a.H + h) * a.W;
 
-  // this tile's flags and the lengths before the chunk
-  const int v0 = tile * kTile + t * kPer;
-  bool f[kPer];
-#pragma unroll
-  for (int k = 0; k < kPer; ++k) f[k] = v0 + k < n_adm && vflag(a, h, v0 + k);
-  const int gl_t = t < a.H ? a.global_lengths[a.layer * a.H + t] : 0;
-  for (int i = t; i < a.H; i += kThreads) s_tot[i] = 0;
-  if (t == 0) {
-    s_pre = 0;
-    s_fail = 0;
-    s_nf = *a.next_free;
-  }
-  __syncthreads();
+  const int nf = *a.next_free;
+  const int gl0 = lens[h];
+  const int gl_t = lane < a.H ? lens[lane] : 0;
+  const int open_page = gl0 % a.page ? bt[gl0 / a.page] : 0;  // the head's last page, partly filled
 
-  // ---- admitted counts of every head, and of this head before the tile ----
-  const int gph = n_adm > 0 ? (n_adm + kCnt - 1) / kCnt : 0;  // count loads per head
-  const int ng = a.H * gph;
-  for (int g0 = t; g0 < ng; g0 += kThreads * kLoads) {
-    int c[kLoads];
-#pragma unroll
-    for (int k = 0; k < kLoads; ++k) {
-      const int g = g0 + k * kThreads;
-      c[k] = g < ng ? count16(a, g / gph, (g % gph) * kCnt, n_adm) : 0;
-    }
-#pragma unroll
-    for (int k = 0; k < kLoads; ++k) {
-      const int g = g0 + k * kThreads;
-      if (g < ng && c[k]) {
-        const int hh = g / gph;
-        atomicAdd(&s_tot[hh], c[k]);
-        if (hh == h && (g % gph) * kCnt < tile * kTile) atomicAdd(&s_pre, c[k]);
-      }
-    }
+  // ---- admitted counts of every head, and of this head before v0 ----------
+  for (int hh = wid; hh < a.H; hh += kWaves) {
+    const int c = wave_sum_int(vcount(a, hh, n_adm, lane, 64));
+    if (lane == 0) s_tot[hh] = c;
   }
+  const int pre = wave_sum_int(v0 > 0 ? vcount(a, h, min(v0, n_adm), t, kThreads) : 0);
+  if (lane == 0) s_wave[wid] = pre;
   __syncthreads();
 
   // ---- the plan (identical in every workgroup) ----------------------------
-  if (a.H <= 64) {
-    if (wid == 0) {
-      int pages = 0;
-      if (lane < a.H) {
-        const int n = s_tot[lane];
-        pages = (gl_t + n + a.page - 1) / a.page - (gl_t + a.page - 1) / a.page;
-        if (n > 0 && (a.W + gl_t + n > a.max_tokens_per_head || lb + (gl_t + n + a.page - 1) / a.page > a.max_pages))
-          s_fail = 1;
-      }
-      const int incl = wave_incl_scan(pages, lane);
-      if (lane < a.H) s_first[lane] = incl - pages;
-      if (lane == 63) {
-        s_total_pages = incl;
-        if ((int64_t)s_nf + incl > a.total_pages) s_fail = 1;
-      }
-    }
-  } else {
-    int carry = 0;
-    for (int h0 = 0; h0 < a.H; h0 += kThreads) {
-      const int hh = h0 + t;
+  if (wid == 0) {
+    int carry = 0, bad = 0;
+    for (int h0 = 0; h0 < a.H; h0 += 64) {
+      const int hh = h0 + lane;
       int pages = 0;
       if (hh < a.H) {
         const int n = s_tot[hh];
-        const int gl = h0 == 0 ? gl_t : a.global_lengths[a.layer * a.H + hh];
+        const int gl = h0 == 0 ? gl_t : lens[hh];
         pages = (gl + n + a.page - 1) / a.page - (gl + a.page - 1) / a.page;
-        if (n > 0 && (a.W + gl + n > a.max_tokens_per_head || lb + (gl + n + a.page - 1) / a.page > a.max_pages))
-          atomicOr(&s_fail, 1);
+        if (n > 0 && (a.W + gl + n > a.max_tokens_per_head || lb + (gl + n + a.page - 1) / a.page > a.max_pages)) bad = 1;
       }
-      int total = 0;
-      const int excl = block_exclusive_scan_256(pages, s_tmp, &total);
-      if (hh < a.H) s_first[hh] = carry + excl;
-      carry += total;
+      const int incl = wave_incl_scan(pages, lane);
+      if (hh == h) s_first = carry + incl - pages;
+      carry += __builtin_amdgcn_readlane(incl, 63);
     }
-    if (t == 0) {
+    bad = __builtin_amdgcn_ballot_w64(bad != 0) != 0;
+    if (lane == 0) {
       s_total_pages = carry;
-      if ((int64_t)s_nf + carry > a.total_pages) s_fail = 1;
+      s_fail = bad || (int64_t)nf + carry > a.total_pages;
     }
   }
   __syncthreads();
@@ -215,79 +154,57 @@ __global__ __launch_bounds__(kThreads) void chunk_admit_kernel(ChunkArgs a) {
   }
   if (fail) return;  // tile 0 of each head has zeroed its column counts
 
-  // ---- this tile: stable compaction and column counts ----------------------
-  const int gl0 = a.global_lengths[a.layer * a.H + h];
+  // ---- this workgroup's steps: stable compaction and column counts ---------
   const int first_new = (gl0 + a.page - 1) / a.page;  // index of the head's first new page
-  const int page0 = s_nf + s_first[h];                  // its page id
-  const int32_t* bt = a.block_table + ((int64_t)a.layer * a.H + h) * a.max_pages + lb;
+  const int page0 = nf + s_first;                       // its page id
   if (tile == 0) {
     const int n_h = s_tot[h];
     const int pages = (gl0 + n_h + a.page - 1) / a.page - first_new;
-    int32_t* row = a.block_table + ((int64_t)a.layer * a.H + h) * a.max_pages + lb;
-    for (int i = t; i < pages; i += kThreads) row[first_new + i] = page0 + i;
+    for (int i = t; i < pages; i += kThreads) bt[first_new + i] = page0 + i;
     if (t == 0) {
       a.adm[h] = n_h;
       a.gl_before[h] = gl0;
       if (h == 0) {
-        *a.next_free_after = s_nf + s_total_pages;
+        *a.next_free_after = nf + s_total_pages;
         *a.abort_flag = 0;
       }
     }
   }
   const int base = a.c0 > 0 ? a.c0 - a.W : 0;  // global position of virtual index 0
-  int cnt = 0;
-#pragma unroll
-  for (int k = 0; k < kPer; ++k) cnt += f[k] ? 1 : 0;
-  const int incl = wave_incl_scan(cnt, lane);
-  if (lane == 63) s_wave[wid] = incl;
-  __syncthreads();
-  int o = incl - cnt, total = 0;
-#pragma unroll
-  for (int w = 0; w < kWaves; ++w) {
-    o += w < wid ? s_wave[w] : 0;
-    total += s_wave[w];
-  }
-  const int before = gl0 + s_pre;
-#pragma unroll
-  for (int k = 0; k < kPer; ++k) {
-    const int v = v0 + k;
-    if (f[k]) {
-      const int j = before + o;  // logical index in the head's global cache
-      const int pi = j / a.page;
-      const int pg = pi < first_new ? bt[pi] : page0 + (pi - first_new);
-      s_src[o] = v;
-      s_dst[o] = (int64_t)pg * a.page + j % a.page;
-      ++o;
-    }
-    // o is now the inclusive count at v within the tile
-    const int pp = base + v + 1;
-    if (v < n_adm && pp > 0 && (pp + a.W - 1) % kBlk == 0) {
-      const int r = (pp + a.W - 1) / kBlk;
-      if (r >= a.r0 && r < a.r0 + a.rchunk) cc[r - a.r0] = before + o;
-    }
-  }
-  __syncthreads();
-  const int chunks = a.D / 8;
   const int64_t ring_base = ((int64_t)a.layer * a.H + h) * a.W;
-  for (int e = t; e < total * chunks; e += kThreads) {
-    const int r = e / chunks, c = e - r * chunks;
-    const int v = s_src[r];
-    u32x4_t kv, vv;
-    if (v < nr) {
-      kv = *(const u32x4_t*)(a.pool_k + (ring_base + v) * a.D + c * 8);
-      vv = *(const u32x4_t*)(a.pool_v + (ring_base + v) * a.D + c * 8);
-    } else {
-      const int64_t off = (int64_t)h * a.kv_sh + (int64_t)(v - nr) * a.kv_ss + c * 8;
-      kv = *(const u32x4_t*)(a.key + off);
-      vv = *(const u32x4_t*)(a.value + off);
+  int before = gl0 + (s_wave[0] + s_wave[1]) + (s_wave[2] + s_wave[3]);
+  for (int v = v0; v < min(n_adm, v0 + a.span * kBlk); v += kBlk) {
+    // the step lies all in the ring or all in the chunk (W is a multiple of 64)
+    const bool in_ring = v < nr;
+    const uint8_t* fl = in_ring ? ring_flags + v : a.mask + (int64_t)h * a.m_sh + (v - nr);
+    const uint64_t adm = __builtin_amdgcn_ballot_w64(v + lane < n_adm && fl[lane] != 0);
+    if (wid == 0) {
+      if (adm >> lane & 1) {
+        const int o = __builtin_popcountll(adm & ((1ull << lane) - 1));
+        const int j = before + o;  // logical index in the head's global cache
+        const int pi = j / a.page;
+        const int pg = pi < first_new ? open_page : page0 + (pi - first_new);
+        s_src[o] = (in_ring ? v : v - nr) + lane;
+        s_dst[o] = (int64_t)pg * a.page + (j - pi * a.page);
+      }
+      const int r = (base + v + a.W) / kBlk;  // the row block whose band starts at this step's second position
+      if (lane == 0 && r >= a.r0 && r < a.r0 + a.rchunk) cc[r - a.r0] = before + (int)(adm & 1);
     }
-    *(u32x4_t*)(a.pool_k + s_dst[r] * a.D + c * 8) = kv;
-    *(u32x4_t*)(a.pool_v + s_dst[r] * a.D + c * 8) = vv;
+    __syncthreads();
+    const int n = __builtin_popcountll(adm);
+    copy_rows2<kThreads>(in_ring ? a.pool_k + ring_base * a.D : a.key + (int64_t)h * a.kv_sh,
+                         in_ring ? a.pool_v + ring_base * a.D : a.value + (int64_t)h * a.kv_sh,
+                         in_ring ? (int64_t)a.D : a.kv_ss, n, a.D, [&](unsigned r) { return s_src[r]; },
+                         [&](unsigned r) { return s_dst[r]; }, a.pool_k, a.pool_v);
+    before += n;
+    __syncthreads();
   }
 }
 
 // After the chunk's attention: ring slot i <- chunk position C - W + i.
-// Grid (head, 64-slot group).
+// Grid (head, 64-slot group); a thread's rows are all requested before the
+// first store (one at a time: 9.2 us for 8 heads of W 1024 with the pre-RoPE
+// keys; 6.6 us).
 __global__ __launch_bounds__(kThreads) void chunk_ring_kernel(ChunkArgs a) {
   if (*a.abort_flag) return;
   const int h = blockIdx.x;
@@ -302,17 +219,13 @@ __global__ __launch_bounds__(kThreads) void chunk_ring_kernel(ChunkArgs a) {
   const int i0 = blockIdx.y * kBlk, i1 = min(n_loc, i0 + kBlk);
   if (i0 >= i1) return;
   const int64_t ring_base = ((int64_t)a.layer * a.H + h) * a.W;
-  const int chunks = a.D / 8;
-  for (int e = threadIdx.x; e < (i1 - i0) * chunks; e += kThreads) {
-    const int i = i0 + e / chunks, c = e % chunks;
-    const int64_t off = (int64_t)h * a.kv_sh + (int64_t)(first + i) * a.kv_ss + c * 8;
-    *(u32x4_t*)(a.pool_k + (ring_base + i) * a.D + c * 8) = *(const u32x4_t*)(a.key + off);
-    *(u32x4_t*)(a.pool_v + (ring_base + i) * a.D + c * 8) = *(const u32x4_t*)(a.value + off);
-    if (a.pre_key && a.local_pre_key) {
-      const int64_t po = (int64_t)h * a.pk_sh + (int64_t)(first + i) * a.pk_ss + c * 8;
-      *(u32x4_t*)(a.local_pre_key + (ring_base + i) * a.D + c * 8) = *(const u32x4_t*)(a.pre_key + po);
-    }
-  }
+  copy_rows2<kThreads>(a.key + (int64_t)h * a.kv_sh, a.value + (int64_t)h * a.kv_sh, a.kv_ss, i1 - i0, a.D,
+                       [&](unsigned r) { return first + i0 + (int)r; }, [&](unsigned r) { return ring_base + i0 + r; },
+                       a.pool_k, a.pool_v);
+  if (a.pre_key && a.local_pre_key)
+    copy_rows1<kThreads>(a.pre_key + (int64_t)h * a.pk_sh, a.pk_ss, i1 - i0, a.D,
+                         [&](unsigned r) { return first + i0 + (int)r; }, [&](unsigned r) { return ring_base + i0 + r; },
+                         a.local_pre_key);
   for (int i = i0 + threadIdx.x; i < i1; i += kThreads)
     a.local_is_global[ring_base + i] = a.mask[(int64_t)h * a.m_sh + first + i] ? 1 : 0;
 }
@@ -384,9 +297,11 @@ extern "C" int wgkv_chunk_cache_update(
   a.column_count = column_count;
   a.r0 = chunk_start / kBlk;
   a.rchunk = (chunk_len + kBlk - 1) / kBlk;
-  const int vl = (chunk_start > 0 ? local_window : 0) + chunk_len;
-  a.ntiles = (vl + kTile - 1) / kTile;
-  a.mask_vec16 = (((uintptr_t)g_mask | (uintptr_t)gm_stride_h) & 15) == 0;
+  // 64-position steps of the admission range, and how many a workgroup takes:
+  // one while the grid is small; more, up to kMaxSpan, where the counting that
+  // every workgroup repeats would outweigh its own steps
+  const int steps = (max(1, vlen(a) - local_window) + kBlk - 1) / kBlk;
+  a.span = min(kMaxSpan, max(1, (int)((int64_t)steps * num_kv_heads / 1024)));
   int32_t* ws = (int32_t*)workspace;
   a.adm = ws;
   a.gl_before = ws + num_kv_heads;
@@ -394,7 +309,7 @@ extern "C" int wgkv_chunk_cache_update(
   a.abort_flag = a.next_free_after + 1;
   hipStream_t st = (hipStream_t)stream;
   if (stage == 0) {
-    hipLaunchKernelGGL(chunk_admit_kernel, dim3(a.ntiles, num_kv_heads), dim3(kThreads), 0, st, a);
+    hipLaunchKernelGGL(chunk_admit_kernel, dim3((steps + a.span - 1) / a.span, num_kv_heads), dim3(kThreads), 0, st, a);
   } else {
     const int groups = (min(local_window, chunk_start + chunk_len) + kBlk - 1) / kBlk;
     hipLaunchKernelGGL(chunk_ring_kernel, dim3(num_kv_heads, groups), dim3(kThreads), 0, st, a);

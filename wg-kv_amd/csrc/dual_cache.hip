@@ -55,38 +55,6 @@ struct AdmitArgs {
   int32_t* abort_flag;
 };
 
-// Copies rows r < n of one K/V pair (source row src(r), pool row dst(r)) with
-// the whole workgroup, 16 bytes per thread and step.  Eight loads per thread
-// are requested before the first store: one load and one store at a time
-// waited for memory once per step (64 us of a 9001-token prompt's 75).
-template <typename Src, typename Dst>
-__device__ __forceinline__ void copy_rows2(const uint16_t* ka, const uint16_t* va, int64_t ss, int n, int D, Src src,
-                                           Dst dst, uint16_t* pool_k, uint16_t* pool_v) {
-  constexpr int U = 4;
-  const unsigned chunks = D / 8;
-  const unsigned total = n * chunks;
-  for (unsigned e0 = threadIdx.x; e0 < total; e0 += kThreads * U) {
-    u32x4_t k[U], v[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const unsigned e = min(e0 + u * kThreads, total - 1);
-      const unsigned r = e / chunks;
-      const int64_t off = (int64_t)src(r) * ss + (e - r * chunks) * 8;
-      k[u] = *(const u32x4_t*)(ka + off);
-      v[u] = *(const u32x4_t*)(va + off);
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const unsigned e = e0 + u * kThreads;
-      if (e >= total) break;
-      const unsigned r = e / chunks;
-      const int64_t off = dst(r) * D + (e - r * chunks) * 8;
-      *(u32x4_t*)(pool_k + off) = k[u];
-      *(u32x4_t*)(pool_v + off) = v[u];
-    }
-  }
-}
-
 // Flags of one count tile of one head (prompts of many tiles only).
 __global__ __launch_bounds__(kThreads) void admit_count_kernel(AdmitArgs a) {
   __shared__ int s_w[kThreads / 64];
@@ -227,7 +195,7 @@ __global__ __launch_bounds__(kThreads) void admit_scatter_kernel(AdmitArgs a) {
   const int64_t base_row = row0 + ((s_w[0] + s_w[1]) + (s_w[2] + s_w[3]));
   const uint16_t* key = a.key + (int64_t)h * a.kv_sh;
   const uint16_t* value = a.value + (int64_t)h * a.kv_sh;
-  copy_rows2(key, value, a.kv_ss, __builtin_popcountll(adm), a.D, [&](unsigned r) { return s_src[r]; },
+  copy_rows2<kThreads>(key, value, a.kv_ss, __builtin_popcountll(adm), a.D, [&](unsigned r) { return s_src[r]; },
              [&](unsigned r) { return base_row + r; }, a.pool_k, a.pool_v);
   // ring part: slot i <- position S - n_loc + i (src/modeling_layers.py:1290-1300)
   const int ring0 = a.S - n_loc;
@@ -235,29 +203,13 @@ __global__ __launch_bounds__(kThreads) void admit_scatter_kernel(AdmitArgs a) {
   if (lo >= hi) return;
   const int64_t slot0 = ((int64_t)a.layer * a.H + h) * a.W + (lo - ring0);
   if (wid == 0 && p >= lo && p < hi) a.local_is_global[slot0 + (p - lo)] = flag ? 1 : 0;
-  copy_rows2(key, value, a.kv_ss, hi - lo, a.D, [&](unsigned r) { return lo + (int)r; },
+  copy_rows2<kThreads>(key, value, a.kv_ss, hi - lo, a.D, [&](unsigned r) { return lo + (int)r; },
              [&](unsigned r) { return slot0 + r; }, a.pool_k, a.pool_v);
   if (a.pre_key && a.local_pre_key) {
     // local_pre_key is (L, H, W, D): its row index equals the pool's ring row
-    const unsigned chunks = a.D / 8, total = (hi - lo) * chunks;
-    const uint16_t* pk = a.pre_key + (int64_t)h * a.pk_sh;
-    constexpr int U = 4;
-    for (unsigned e0 = t; e0 < total; e0 += kThreads * U) {
-      u32x4_t v[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const unsigned e = min(e0 + u * kThreads, total - 1);
-        const unsigned r = e / chunks;
-        v[u] = *(const u32x4_t*)(pk + (int64_t)(lo + (int)r) * a.pk_ss + (e - r * chunks) * 8);
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const unsigned e = e0 + u * kThreads;
-        if (e >= total) break;
-        const unsigned r = e / chunks;
-        *(u32x4_t*)(a.local_pre_key + (slot0 + r) * a.D + (e - r * chunks) * 8) = v[u];
-      }
-    }
+    copy_rows1<kThreads>(a.pre_key + (int64_t)h * a.pk_sh, a.pk_ss, hi - lo, a.D,
+                         [&](unsigned r) { return lo + (int)r; }, [&](unsigned r) { return slot0 + r; },
+                         a.local_pre_key);
   }
 }
 

@@ -140,13 +140,77 @@ WGKV_DEVICE int count_flags(const uint8_t* m, int lo, int hi, int t, int n) {
   if (t < head) c += p[t] != 0;
   if (t < tail) c += m[hi - tail + t] != 0;
   const u32x4_t* v = (const u32x4_t*)(p + head);
-  for (int g = t; g < groups; g += n) {
-    const u32x4_t w = v[g];
+  constexpr int U = 4;  // loads in flight
+  for (int g0 = t; g0 < groups; g0 += n * U) {
+    u32x4_t w[U];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)  // bit 7 of each nonzero byte
-      c += __builtin_popcount((((w[i] & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w[i]) & 0x80808080u);
+    for (int u = 0; u < U; ++u) w[u] = v[min(g0 + u * n, groups - 1)];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      int k = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)  // bit 7 of each nonzero byte
+        k += __builtin_popcount((((w[u][i] & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w[u][i]) & 0x80808080u);
+      c += g0 + u * n < groups ? k : 0;
+    }
   }
   return c;
+}
+
+// Copies rows r < n of one K/V pair (source row src(r), pool row dst(r)) with
+// the whole workgroup of kThreads, 16 bytes per thread and step.  Eight loads per thread
+// are requested before the first store: one load and one store at a time
+// waited for memory once per step (64 us of a 9001-token prompt's 75).
+template <int kThreads, typename Src, typename Dst>
+WGKV_DEVICE void copy_rows2(const uint16_t* ka, const uint16_t* va, int64_t ss, int n, int D, Src src, Dst dst,
+                            uint16_t* pool_k, uint16_t* pool_v) {
+  constexpr int U = 4;
+  const unsigned chunks = D / 8;
+  const unsigned total = n * chunks;
+  for (unsigned e0 = threadIdx.x; e0 < total; e0 += kThreads * U) {
+    u32x4_t k[U], v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const unsigned e = min(e0 + u * kThreads, total - 1);
+      const unsigned r = e / chunks;
+      const int64_t off = (int64_t)src(r) * ss + (e - r * chunks) * 8;
+      k[u] = *(const u32x4_t*)(ka + off);
+      v[u] = *(const u32x4_t*)(va + off);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const unsigned e = e0 + u * kThreads;
+      if (e >= total) break;
+      const unsigned r = e / chunks;
+      const int64_t off = dst(r) * D + (e - r * chunks) * 8;
+      *(u32x4_t*)(pool_k + off) = k[u];
+      *(u32x4_t*)(pool_v + off) = v[u];
+    }
+  }
+}
+
+// The same for one array.
+template <int kThreads, typename Src, typename Dst>
+WGKV_DEVICE void copy_rows1(const uint16_t* a, int64_t ss, int n, int D, Src src, Dst dst, uint16_t* to) {
+  constexpr int U = 4;
+  const unsigned chunks = D / 8;
+  const unsigned total = n * chunks;
+  for (unsigned e0 = threadIdx.x; e0 < total; e0 += kThreads * U) {
+    u32x4_t v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const unsigned e = min(e0 + u * kThreads, total - 1);
+      const unsigned r = e / chunks;
+      v[u] = *(const u32x4_t*)(a + (int64_t)src(r) * ss + (e - r * chunks) * 8);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const unsigned e = e0 + u * kThreads;
+      if (e >= total) break;
+      const unsigned r = e / chunks;
+      *(u32x4_t*)(to + dst(r) * D + (e - r * chunks) * 8) = v[u];
+    }
+  }
 }
 
 #define WGKV_HIP_CHECK(expr)                       \
