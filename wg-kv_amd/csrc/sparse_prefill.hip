@@ -445,10 +445,11 @@ __global__ __launch_bounds__(128 * HPW) void sparse_prefill_kernel(PrefillArgs a
               sc[kt][rt][i] = kk < lim ? sc[kt][rt][i] : -INFINITY;
             }
         }
-        float mx = -INFINITY;
+        float mx = sc[0][rt][0];
   #pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-          mx = fmax_ieee(mx, fmax_ieee(fmax_ieee(sc[kt][rt][0], sc[kt][rt][1]), fmax_ieee(sc[kt][rt][2], sc[kt][rt][3])));
+        for (int e = 1; e < 15; e += 2)
+          mx = fmax_ieee(fmax_ieee(mx, sc[e >> 2][rt][e & 3]), sc[(e + 1) >> 2][rt][(e + 1) & 3]);
+        mx = fmax_ieee(mx, sc[3][rt][3]);
         mxs[rt] = mx;  // this lane's 16 keys of the row
       }
       // A row needs the rescale iff one of its four lanes' maxima exceeds
