@@ -575,17 +575,24 @@ hipError_t launch(const PrefillArgs& a, hipStream_t st, bool chunked) {
 
 // Query heads per workgroup: the largest of 4, 2, 1 that divides G and lets
 // every wave load whole 1 KB blocks of a tile (2 * HPW waves, D / 8 blocks:
-// at most 2 heads at D = 32).  G = 3 then takes one head per workgroup.
-int heads_per_wg(int head_dim, int G) {
-  const int cap = head_dim == 32 ? 2 : 4;
-  for (int h = cap; h > 1; h >>= 1)
-    if (G % h == 0) return h;
-  return 1;
+// at most 2 heads at D = 32); G = 3 then takes one head per workgroup.  Halved
+// while the smaller workgroups would still get a CU each: a short prompt's
+// time is its longest item's, and a SIMD with one wave runs a tile sooner than
+// one that two waves share, which outweighs loading each K/V tile once per
+// half of the heads.  8 KV heads, G = 4, W 1024, 20 % admitted, 4 / 2 / 1
+// heads per workgroup: 500 tokens (64 items of 4 heads) 22.3 / 18.5 / 18.1 us,
+// 777 (104) 30.2 / 25.4 / 27.3, 1024 (128) 37.4 / 31.4 / 32.4, 2048 (256)
+// 48.3 / 64.4 / 65.8.
+int heads_per_wg(int head_dim, int G, int64_t rows) {
+  int h = head_dim == 32 ? 2 : 4;
+  while (G % h) h >>= 1;
+  while (h > 1 && rows * (G / h) * 2 <= cu_count()) h >>= 1;
+  return h;
 }
 
 hipError_t launch_any(PrefillArgs& a, hipStream_t st, int head_dim, int G, bool chunked) {
   a.G = G;
-  const int hpw = heads_per_wg(head_dim, G);
+  const int hpw = heads_per_wg(head_dim, G, (int64_t)a.R * a.B * a.Hkv);
   if (head_dim == 128)
     return hpw == 1 ? launch<128, 1>(a, st, chunked) : hpw == 2 ? launch<128, 2>(a, st, chunked)
                     : launch<128, 4>(a, st, chunked);
