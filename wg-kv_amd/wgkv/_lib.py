@@ -237,6 +237,13 @@ def check(status, where):
     raise WGKVError(status, where)
 
 
+# torch's current stream of a device as an integer, without building a Stream
+# object (2 us of a call's host time); None where torch does not have it
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_handle(device=None):
     """hipStream_t of torch's current stream on ``device``."""
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    if _raw_stream is not None and type(device) is torch.device and device.index is not None:
+        return _raw_stream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream

@@ -20,8 +20,9 @@ _retired = []  # replaced workspaces, kept for graphs captured with their addres
 
 
 def _dev_key(device):
-    dev = torch.device(device)
-    return dev, (dev.index if dev.index is not None else torch.cuda.current_device())
+    dev = device if type(device) is torch.device else torch.device(device)
+    index = dev.index
+    return dev, (index if index is not None else torch.cuda.current_device())
 
 
 def workspace(device, nbytes):
@@ -60,6 +61,12 @@ def _require_cuda(*tensors):
             raise ValueError("wgkv kernels take device tensors (no CPU fallback)")
 
 
+# The wrappers below are a large part of a small call's time (a batch-1 decode
+# kernel runs ~11 us): they read each tensor's shape and strides once, pass
+# whole tensors' addresses instead of slicing them, and leave to the C ABI what
+# it checks itself.
+
+
 # ---------------------------------------------------------------------------
 # kernel (2): ragged paged decode attention
 # ---------------------------------------------------------------------------
@@ -68,16 +75,20 @@ def _validate_decode(q, k_cache, v_cache, cache_seqlens, block_table):
     if q.dim() != 4 or q.shape[1] != 1:
         raise AssertionError("q must be (batch, 1, num_query_heads, head_size)")
     B, _, Hq, D = q.shape
-    if cache_seqlens.dim() != 2 or cache_seqlens.shape[0] != B:
+    sl_shape = cache_seqlens.shape
+    if len(sl_shape) != 2 or sl_shape[0] != B:
         raise AssertionError("cache_seqlens must be (batch, num_kv_heads)")
-    Hkv = cache_seqlens.shape[1]
+    Hkv = sl_shape[1]
     if Hq % Hkv:
         raise AssertionError("num_query_heads must be a multiple of num_kv_heads")
-    if block_table.dim() != 3 or block_table.shape[:2] != (B, Hkv):
+    bt_shape = block_table.shape
+    if len(bt_shape) != 3 or bt_shape[0] != B or bt_shape[1] != Hkv:
         raise AssertionError("block_table must be (batch, num_kv_heads, max_blocks)")
-    if k_cache.dim() != 3 or k_cache.shape != v_cache.shape or k_cache.shape[2] != D:
+    k_shape = k_cache.shape
+    if len(k_shape) != 3 or k_shape != v_cache.shape or k_shape[2] != D:
         raise AssertionError("k_cache/v_cache must be (num_blocks, block_size, head_size)")
-    if q.dtype != torch.bfloat16 or k_cache.dtype != torch.bfloat16 or v_cache.dtype != torch.bfloat16:
+    bf16 = torch.bfloat16
+    if q.dtype != bf16 or k_cache.dtype != bf16 or v_cache.dtype != bf16:
         raise TypeError("This kernel only supports BF16 inputs for q, k_cache, and v_cache.")
     if cache_seqlens.dtype != torch.int32 or block_table.dtype != torch.int32:
         raise TypeError("cache_seqlens and block_table must be int32")
@@ -88,29 +99,35 @@ def paged_decode_attn(q, k_cache, v_cache, cache_seqlens, block_table, softmax_s
     """Decode attention over paged per-head caches; returns (B, 1, Hq, D) bf16."""
     B, Hq, Hkv, D = _validate_decode(q, k_cache, v_cache, cache_seqlens, block_table)
     _require_cuda(q, k_cache, v_cache, cache_seqlens, block_table)
-    q3 = q[:, 0]
-    if q3.stride(2) != 1:
-        q3 = q3.contiguous()
+    qs = q.stride()
+    if qs[3] != 1:
+        q = q.contiguous()
+        qs = q.stride()
     if not (k_cache.is_contiguous() and v_cache.is_contiguous()):
         raise ValueError("k_cache/v_cache must be contiguous")
     sl = cache_seqlens if cache_seqlens.stride(1) == 1 else cache_seqlens.contiguous()
-    bt = block_table if block_table.stride(2) == 1 else block_table.contiguous()
+    bt = block_table
+    bs = bt.stride()
+    if bs[2] != 1:
+        bt = bt.contiguous()
+        bs = bt.stride()
+    dev = q.device
     if out is None:
-        out = torch.empty(B, 1, Hq, D, dtype=torch.bfloat16, device=q.device)
-    o3 = out[:, 0]
-    L = _lib.lib()
-    ws = decode_workspace(q.device)
-    st = L.wgkv_paged_decode_attn(
-        _ptr(q3), q3.stride(0), q3.stride(1),
-        _ptr(k_cache), _ptr(v_cache), k_cache.shape[0], k_cache.shape[1],
-        _ptr(sl), sl.stride(0),
-        _ptr(bt), bt.stride(0), bt.stride(1), bt.shape[2],
-        _ptr(o3), o3.stride(0), o3.stride(1),
+        out = torch.empty(B, 1, Hq, D, dtype=torch.bfloat16, device=dev)
+    os = out.stride()
+    ws = decode_workspace(dev)
+    st = _lib.lib().wgkv_paged_decode_attn(
+        q.data_ptr(), qs[0], qs[2],
+        k_cache.data_ptr(), v_cache.data_ptr(), k_cache.shape[0], k_cache.shape[1],
+        sl.data_ptr(), sl.stride(0),
+        bt.data_ptr(), bs[0], bs[1], bt.shape[2],
+        out.data_ptr(), os[0], os[2],
         B, Hq, Hkv, D,
         float(softmax_scale),
-        _ptr(ws), ws.numel(),
-        _lib.stream_handle(q.device))
-    _lib.check(st, "wgkv_paged_decode_attn")
+        ws.data_ptr(), ws.numel(),
+        _lib.stream_handle(dev))
+    if st:
+        _lib.check(st, "wgkv_paged_decode_attn")
     return out
 
 
@@ -160,7 +177,7 @@ def generate_sparse_indices(g_mask, local_window_size, batch_size, num_kv_heads,
         raise AssertionError("g_mask must be (batch, num_kv_heads, seq_len)")
     _require_cuda(g_mask)
     dev = g_mask.device
-    m = g_mask if g_mask.dtype == torch.uint8 else g_mask.to(torch.bool).view(torch.uint8)
+    m = _u8(g_mask)
     if m.stride(2) != 1:
         m = m.contiguous()
     R = (seq_len + block_size - 1) // block_size
@@ -170,7 +187,7 @@ def generate_sparse_indices(g_mask, local_window_size, batch_size, num_kv_heads,
     block_offset = torch.empty(1, 1, R, P + 1, **i32)
     column_count = torch.empty(batch_size, num_kv_heads, R, **i32)
     column_index = torch.empty(batch_size, num_kv_heads, 1, seq_len, **i32)
-    column_total = torch.empty(batch_size, num_kv_heads, **i32)
+    column_total = torch.empty(batch_size, num_kv_heads, **i32) if exact_width else None
     st = _lib.lib().wgkv_build_prefill_meta(
         _ptr(m), m.stride(0), m.stride(1),
         batch_size, num_kv_heads, seq_len, local_window_size, block_size,
@@ -188,7 +205,9 @@ def generate_sparse_indices(g_mask, local_window_size, batch_size, num_kv_heads,
 # kernel (1), cache half: prefill admission and the decode-step append
 # ---------------------------------------------------------------------------
 def _u8(mask):
-    return mask if mask.dtype == torch.uint8 else mask.to(torch.bool).view(torch.uint8)
+    if mask.dtype == torch.uint8:
+        return mask
+    return (mask if mask.dtype == torch.bool else mask.to(torch.bool)).view(torch.uint8)
 
 
 def prefill_admit(cache, layer, key, value, g_mask, pre_key=None):
@@ -203,7 +222,8 @@ def prefill_admit(cache, layer, key, value, g_mask, pre_key=None):
     if m.stride(1) != 1:
         m = m.contiguous()
     L = _lib.lib()
-    ws = workspace(key.device, L.wgkv_prefill_admit_workspace_bytes(H, S))
+    dev = key.device
+    ws = workspace(dev, L.wgkv_prefill_admit_workspace_bytes(H, S))
     lpk = cache.local_pre_key if (pre_key is not None and cache.local_pre_key is not None) else None
     st = L.wgkv_prefill_admit(
         _ptr(key), _ptr(value), key.stride(0), key.stride(1),
@@ -215,7 +235,7 @@ def prefill_admit(cache, layer, key, value, g_mask, pre_key=None):
         _ptr(cache.block_pool_k), _ptr(cache.block_pool_v), _ptr(cache.block_table), cache.block_table.shape[2],
         _ptr(cache.global_lengths), _ptr(cache.local_is_global.view(torch.uint8)), _ptr(lpk),
         _ptr(cache.next_free_block_dev), _ptr(cache.status),
-        _ptr(ws), ws.numel(), _lib.stream_handle(key.device))
+        _ptr(ws), ws.numel(), _lib.stream_handle(dev))
     _lib.check(st, "wgkv_prefill_admit")
 
 
@@ -295,29 +315,35 @@ def sparse_attn_func(q, k, v, block_count, block_offset, column_count, column_in
     if k.stride() != v.stride():
         raise ValueError("k and v must share strides")
     _require_cuda(q, k, v, block_count, block_offset, column_count, column_index)
-    if q.stride(3) != 1 or k.stride(3) != 1:
+    qs, ks = q.stride(), k.stride()
+    if qs[3] != 1 or ks[3] != 1:
         raise ValueError("head_dim must be contiguous")
     R = (S + 63) // 64
-    if block_count.numel() != R or column_count.shape != (B, Hkv, R):
+    if block_count.numel() != R or block_offset.numel() % R or column_count.shape != (B, Hkv, R):
         raise AssertionError("metadata does not match (batch, heads, seq) with block 64")
     if softmax_scale is None:
         softmax_scale = D ** -0.5
-    bc = block_count.reshape(R).contiguous()
-    bo = block_offset.reshape(R, -1).contiguous()
+    bc = block_count.contiguous()  # R counts
+    bo = block_offset.contiguous()  # R rows
     cc = column_count.contiguous()
     ci = column_index
-    if ci.stride(-1) != 1:
+    cs = ci.stride()
+    if cs[-1] != 1:
         ci = ci.contiguous()
+        cs = ci.stride()
+    dev = q.device
     if out is None:
-        out = torch.empty(B, S, Hq, D, dtype=torch.bfloat16, device=q.device)
+        out = torch.empty(B, S, Hq, D, dtype=torch.bfloat16, device=dev)
+    os = out.stride()
     st = _lib.lib().wgkv_sparse_prefill_attn(
-        _ptr(q), q.stride(0), q.stride(1), q.stride(2),
-        _ptr(k), _ptr(v), k.stride(0), k.stride(1), k.stride(2),
-        _ptr(out), out.stride(0), out.stride(1), out.stride(2),
-        _ptr(bc), _ptr(bo), bo.shape[1],
-        _ptr(cc), _ptr(ci), ci.stride(0), ci.stride(1),
-        B, S, Hq, Hkv, D, 64, float(softmax_scale), _lib.stream_handle(q.device))
-    _lib.check(st, "wgkv_sparse_prefill_attn")
+        q.data_ptr(), qs[0], qs[1], qs[2],
+        k.data_ptr(), v.data_ptr(), ks[0], ks[1], ks[2],
+        out.data_ptr(), os[0], os[1], os[2],
+        bc.data_ptr(), bo.data_ptr(), bo.numel() // R,
+        cc.data_ptr(), ci.data_ptr(), cs[0], cs[1],
+        B, S, Hq, Hkv, D, 64, float(softmax_scale), _lib.stream_handle(dev))
+    if st:
+        _lib.check(st, "wgkv_sparse_prefill_attn")
     return out
 
 
