@@ -671,18 +671,6 @@ __global__ void zero_counters_kernel(int* c, int n) {
   if (i < n) c[i] = 0;
 }
 
-int cu_count() {
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cached[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cached[dev] = n;
-  }
-  return cached[dev];
-}
-
 template <int D, int G, int NW>
 hipError_t launch_nw(DecodeArgs a, hipStream_t st) {
   const int BH = a.B * a.Hkv;

@@ -98,21 +98,22 @@ __device__ __forceinline__ float score_of(const GateArgs& a, float z, float b2) 
   return g;
 }
 
-// End of a 64-token tile: lane (n, kq) holds partial logits of tokens
+// End of a tile of 16 * MT tokens: lane (n, kq) holds partial logits of tokens
 // mt*16 + 4*kq + i over its columns; sum over the 16 lanes of each row, then
 // over the 4 waves, and apply b2, sigmoid, clamp and threshold.
-__device__ __forceinline__ void finish_tile(const GateArgs& a, const float (&logit)[4][4], float (*s_part)[kTok],
+template <int MT>
+__device__ __forceinline__ void finish_tile(const GateArgs& a, const float (&logit)[MT][4], float (*s_part)[MT * 16],
                                             int lane, int wid, int b, int h, int s0) {
   const int n = lane & 15, kq = lane >> 4;
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
+  for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const float v = row_sum16(logit[mt][i]);
       if (n == 0) s_part[wid][mt * 16 + 4 * kq + i] = v;
     }
   __syncthreads();
-  if (threadIdx.x < kTok) {
+  if (threadIdx.x < MT * 16) {
     const int m = threadIdx.x;
     const int s = s0 + m;
     if (s < a.S) {
@@ -242,7 +243,7 @@ __global__ __launch_bounds__(kThreads) void gate_kernel(GateArgs a) {
         }
     }
   }
-  finish_tile(a, logit, s_part, lane, wid, b, h, s0);
+  finish_tile<4>(a, logit, s_part, lane, wid, b, h, s0);
 }
 
 // Few tokens (decode steps, S <= kSmallTok).  The hidden columns of a head
@@ -525,8 +526,8 @@ __global__ void gate_pack_kernel(const float* __restrict__ w1, const float* wn0,
   }
 }
 
-// One workgroup = 64 tokens of one (batch, KV head), as gate_kernel.  The
-// inputs are read 16 bytes per lane (a wave load covers 64 / (D/8) rows), the
+// One workgroup = 16 * MT tokens (64 or 32) of one (batch, KV head), as
+// gate_kernel.  The inputs are read 16 bytes per lane (a wave load covers 64 / (D/8) rows), the
 // row norms reduced over the D/8 lanes of a row, and y goes to LDS as bf16
 // (rows padded by 16 bytes: the 16 rows of a fragment read start 16 bytes
 // apart modulo 256).  Wave w takes 16-column tiles w, w+4, ... in groups of
@@ -535,7 +536,7 @@ __global__ void gate_pack_kernel(const float* __restrict__ w1, const float* wn0,
 // Two waves per SIMD (two workgroups per CU) hide each other's loads and
 // GELU epilogues.  fp32 parameters only (PREC 0, three planes); bf16
 // parameters run gate_bf16p_kernel.
-template <int D, int NIN, int PREC>
+template <int D, int NIN, int PREC, int MT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void gate_bf16_kernel(GateArgs a, const u32x4_t* __restrict__ packed) {
   static_assert(PREC == 0, "three planes: fp32 parameters (bf16 parameters run gate_bf16p_kernel)");
   constexpr int NP = planes_of(PREC);
@@ -544,16 +545,18 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   constexpr int LDY = K + 8;     // LDS row stride (bf16)
   constexpr int LPR = D / 8;     // lanes per input row
   constexpr int RPL = 64 / LPR;  // rows per wave load
-  constexpr int NLD = 16 / RPL;  // wave loads per input for the wave's 16 tokens
-  __shared__ __attribute__((aligned(16))) uint16_t ys[kTok * LDY];
-  __shared__ float s_part[4][kTok];
+  constexpr int TOK = 16 * MT;   // tokens per workgroup
+  constexpr int TPW = 4 * MT;    // tokens a wave normalises
+  constexpr int NLD = TPW / RPL; // wave loads per input for them
+  __shared__ __attribute__((aligned(16))) uint16_t ys[TOK * LDY];
+  __shared__ float s_part[4][TOK];
   if (inactive(a)) return;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int nbh = a.B * a.H;
   const int lid = blockIdx.x + blockIdx.y * gridDim.x;  // XCD-aware order, as gate_kernel
   const int bh = lid % nbh, tile = lid / nbh;
   const int b = bh / a.H, h = bh - b * a.H;
-  const int s0 = tile * kTok;
+  const int s0 = tile * TOK;
 
   // ---- normalised inputs -> LDS (bf16) ------------------------------------
   {
@@ -563,7 +566,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     for (int i = 0; i < NIN; ++i)
 #pragma unroll
       for (int u = 0; u < NLD; ++u) {
-        const int s = min(s0 + wid * 16 + u * RPL + lane / LPR, a.S - 1);  // rows past S are computed and discarded
+        const int s = min(s0 + wid * TPW + u * RPL + lane / LPR, a.S - 1);  // rows past S are computed and discarded
         const uint16_t* row = (const uint16_t*)a.in[i] + (int64_t)b * a.sb[i] + (int64_t)h * a.sh[i] + (int64_t)s * a.ss[i];
         v[i][u] = *(const u32x4_t*)(row + c * 8);
       }
@@ -590,7 +593,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
           for (int e = 0; e < 4; ++e) y[e] = pack_bf16x2(f[2 * e] * scale, f[2 * e + 1] * scale);  // cast back to bf16 (:128)
         }
-        const int m = wid * 16 + u * RPL + lane / LPR;
+        const int m = wid * TPW + u * RPL + lane / LPR;
         *(u32x4_t*)(&ys[m * LDY + i * D + c * 8]) = y;
       }
   }
@@ -602,18 +605,18 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   const u32x4_t* ph = packed + (int64_t)h * ntot * KS * NP * 64 + lane;
   const float* b1h = a.b1 + (int64_t)h * a.inner;
   const float* w2h = a.w2 + (int64_t)h * a.inner;
-  float logit[4][4];
+  float logit[MT][4];
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
+  for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
     for (int i = 0; i < 4; ++i) logit[mt][i] = 0.f;
   for (int t0 = wid; t0 < ntot; t0 += 16) {
     int tj[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) tj[j] = t0 + 4 * j < ntot ? t0 + 4 * j : t0;  // out-of-range tiles recompute t0, skipped below
-    f32x4_t c[4][4];
+    f32x4_t c[MT][4];
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int j = 0; j < 4; ++j) c[mt][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
     {
@@ -630,14 +633,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         for (int j = 0; j < 4; ++j)
 #pragma unroll
           for (int p = 0; p < NP; ++p) bn[j][p] = ph[(((int64_t)tj[j] * KS + ks + 1) * NP + p) * 64];
-      bf16x8_t ax[4];
+      bf16x8_t ax[MT];
 #pragma unroll
-      for (int mt = 0; mt < 4; ++mt)
+      for (int mt = 0; mt < MT; ++mt)
         ax[mt] = __builtin_bit_cast(bf16x8_t, *(const u32x4_t*)(&ys[(mt * 16 + n) * LDY + ks * 32 + kg * 8]));
 #pragma unroll
       for (int p = NP - 1; p >= 0; --p)  // smallest plane first
 #pragma unroll
-        for (int mt = 0; mt < 4; ++mt)
+        for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
           for (int j = 0; j < 4; ++j)
             c[mt][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ax[mt], __builtin_bit_cast(bf16x8_t, bw[j][p]), c[mt][j], 0, 0, 0);
@@ -654,7 +657,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
       const int col = tj[j] * 16 + n;
       const float bias = b1h[col], wo = w2h[col];
 #pragma unroll
-      for (int mt = 0; mt < 4; ++mt)
+      for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const float z = layer_out(c[mt][j][i], bias, PREC);
@@ -662,7 +665,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         }
     }
   }
-  finish_tile(a, logit, s_part, lane, wid, b, h, s0);
+  finish_tile<MT>(a, logit, s_part, lane, wid, b, h, s0);
 }
 
 // ---- one weight plane (bf16 parameters) -----------------------------------
@@ -679,19 +682,20 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 // The weight fragments are requested PQ k-steps ahead, across group
 // boundaries, and the first group's, with the activation table and the norm
 // weights, before the inputs.
-template <int D, int NIN>
+template <int D, int NIN, int MT>
 struct TileInputs {
   static constexpr int LPR = D / 8;     // lanes per input row
   static constexpr int RPL = 64 / LPR;  // rows per wave load
-  static constexpr int NLD = 16 / RPL;  // wave loads per input for the wave's 16 tokens
+  static constexpr int TPW = 4 * MT;     // tokens a wave normalises
+  static constexpr int NLD = TPW / RPL;  // wave loads per input for them
   u32x4_t v[NIN][NLD];
   f32x4_t wn[NIN][2];
 };
 
-template <int D, int NIN>
+template <int D, int NIN, int MT>
 __device__ __forceinline__ void load_tile_inputs(const GateArgs& a, int b, int h, int s0, int lane, int wid,
-                                                 TileInputs<D, NIN>& t) {
-  using T = TileInputs<D, NIN>;
+                                                 TileInputs<D, NIN, MT>& t) {
+  using T = TileInputs<D, NIN, MT>;
   const int c = lane % T::LPR;
   if (a.rms)
 #pragma unroll
@@ -703,7 +707,7 @@ __device__ __forceinline__ void load_tile_inputs(const GateArgs& a, int b, int h
   for (int i = 0; i < NIN; ++i)
 #pragma unroll
     for (int u = 0; u < T::NLD; ++u) {
-      const int s = min(s0 + wid * 16 + u * T::RPL + lane / T::LPR, a.S - 1);  // rows past S are computed and discarded
+      const int s = min(s0 + wid * T::TPW + u * T::RPL + lane / T::LPR, a.S - 1);  // rows past S are computed and discarded
       const uint16_t* row = (const uint16_t*)a.in[i] + (int64_t)b * a.sb[i] + (int64_t)h * a.sh[i] + (int64_t)s * a.ss[i];
       t.v[i][u] = *(const u32x4_t*)(row + c * 8);
     }
@@ -711,10 +715,10 @@ __device__ __forceinline__ void load_tile_inputs(const GateArgs& a, int b, int h
 
 // y = bf16(x * rsqrt(mean(x^2) + 1e-6)) (:128), times the bf16 norm weight
 // rounded to bf16, as gate_bf16_kernel with bf16 parameters.
-template <int D, int NIN, int LDY>
-__device__ __forceinline__ void store_tile_inputs(const GateArgs& a, int lane, int wid, const TileInputs<D, NIN>& t,
+template <int D, int NIN, int MT, int LDY>
+__device__ __forceinline__ void store_tile_inputs(const GateArgs& a, int lane, int wid, const TileInputs<D, NIN, MT>& t,
                                                   uint16_t* ys) {
-  using T = TileInputs<D, NIN>;
+  using T = TileInputs<D, NIN, MT>;
   const int c = lane % T::LPR;
 #pragma unroll
   for (int i = 0; i < NIN; ++i)
@@ -743,21 +747,22 @@ __device__ __forceinline__ void store_tile_inputs(const GateArgs& a, int lane, i
 #pragma unroll
         for (int e = 0; e < 4; ++e) y[e] = pack_bf16x2(wv[2 * e] * bf16lo(y[e]), wv[2 * e + 1] * bf16hi(y[e]));
       }
-      const int m = wid * 16 + u * T::RPL + lane / T::LPR;
+      const int m = wid * T::TPW + u * T::RPL + lane / T::LPR;
       *(u32x4_t*)(&ys[m * LDY + i * D + c * 8]) = y;
     }
 }
 
-template <int D, int NIN, int PREC>
+template <int D, int NIN, int PREC, int MT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void gate_bf16p_kernel(GateArgs a, const u32x4_t* __restrict__ packed) {
   static_assert(PREC == 1 || PREC == 2, "one plane: bf16 parameters");
   constexpr int K = NIN * D;
   constexpr int KS = K / 32;
+  constexpr int TOK = 16 * MT;
   constexpr int LDY = K + 8;
   constexpr int NTAB = kActTab / 8;                      // 16-byte slices of the table
   constexpr int TPT = (NTAB + kThreads - 1) / kThreads;  // per thread
-  __shared__ __attribute__((aligned(16))) uint16_t ys[kTok * LDY];
-  __shared__ float s_part[4][kTok];
+  __shared__ __attribute__((aligned(16))) uint16_t ys[TOK * LDY];
+  __shared__ float s_part[4][TOK];
   __shared__ __attribute__((aligned(16))) uint16_t s_act[kActTab];
   if (inactive(a)) return;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -765,7 +770,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   const int lid = blockIdx.x + blockIdx.y * gridDim.x;  // XCD-aware order, as gate_kernel
   const int bh = lid % nbh, tile = lid / nbh;
   const int b = bh / a.H, h = bh - b * a.H;
-  const int s0 = tile * kTok;
+  const int s0 = tile * TOK;
   const int n = lane & 15, kg = lane >> 4;
   const int ntot = a.inner / 16;
   const u32x4_t* ph = packed + (int64_t)h * ntot * KS * 64 + lane;
@@ -796,20 +801,20 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 
   // ---- normalised inputs -> LDS -------------------------------------------
   {
-    TileInputs<D, NIN> in;
-    load_tile_inputs<D, NIN>(a, b, h, s0, lane, wid, in);
+    TileInputs<D, NIN, MT> in;
+    load_tile_inputs<D, NIN, MT>(a, b, h, s0, lane, wid, in);
 #pragma unroll
     for (int r = 0; r < TPT; ++r) {
       const int i = threadIdx.x + r * kThreads;
       if (i < NTAB) ((u32x4_t*)s_act)[i] = tab_r[r];
     }
-    store_tile_inputs<D, NIN, LDY>(a, lane, wid, in, ys);
+    store_tile_inputs<D, NIN, MT, LDY>(a, lane, wid, in, ys);
   }
   __syncthreads();
 
-  float logit[4][4];
+  float logit[MT][4];
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
+  for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
     for (int i = 0; i < 4; ++i) logit[mt][i] = 0.f;
   for (int g = 0; g < ng; ++g) {
@@ -823,9 +828,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
       bo[jj] = b1h[col];
       wo[jj] = w2h[col];
     }
-    f32x4_t c[4][TG];
+    f32x4_t c[MT][TG];
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int jj = 0; jj < TG; ++jj) c[mt][jj] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
     // the A fragments are the same for every group: an opaque base keeps the
@@ -834,9 +839,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     asm volatile("" : "+v"(abase));
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      bf16x8_t ax[4];
+      bf16x8_t ax[MT];
 #pragma unroll
-      for (int mt = 0; mt < 4; ++mt)
+      for (int mt = 0; mt < MT; ++mt)
         ax[mt] = __builtin_bit_cast(bf16x8_t, *(const u32x4_t*)(&ys[mt * 16 * LDY + abase + ks * 32]));
       // the slot's next k-step: this group's ks + PQ, else the next group's
       const int slot = ks % PQ;
@@ -847,18 +852,18 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         bq[slot][jj] = ks + PQ < KS ? ph[((int64_t)tn[jj] * KS + ks + PQ) * 64] : ph[((int64_t)tx[jj] * KS + ks + PQ - KS) * 64];
       }
 #pragma unroll
-      for (int mt = 0; mt < 4; ++mt)
+      for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int jj = 0; jj < TG; ++jj)
           c[mt][jj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ax[mt], __builtin_bit_cast(bf16x8_t, bcur[jj]), c[mt][jj], 0, 0, 0);
     }
-    // the group's 64 values of this lane as 32 bf16 pairs (rows i, i+1 of the
+    // the group's 16 * MT values of this lane as bf16 pairs (rows i, i+1 of the
     // lane's column in tile jj): the layer outputs z and their table entries;
     // dmax = the largest table offset (offsets >= kActBytes lie outside)
-    uint32_t zz[32], tvp[32];
+    uint32_t zz[8 * MT], tvp[8 * MT];
     u16x2_t dmax = {0, 0};
 #pragma unroll
-    for (int p = 0; p < 32; ++p) {
+    for (int p = 0; p < 8 * MT; ++p) {
       const int mt = p >> 3, jj = (p >> 1) & 3, i = (p & 1) * 2;
       uint32_t z2;
       if (PREC == 1) {
@@ -881,7 +886,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     }
     if (max(dmax.x, dmax.y) >= kActBytes) {  // rare: some value lies outside the table
 #pragma unroll
-      for (int p = 0; p < 32; ++p) {
+      for (int p = 0; p < 8 * MT; ++p) {
         const u16x2_t zv = __builtin_bit_cast(u16x2_t, zz[p]);
         const u16x2_t d2 = (u16x2_t)(zv << 1) - (u16x2_t)kActBias2;
         if (d2.x >= kActBytes) tvp[p] = (tvp[p] & 0xffff0000u) | (__float_as_uint(activation(bf16lo(zz[p]), a.act, PREC)) >> 16);
@@ -893,7 +898,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     for (int jj = 0; jj < TG; ++jj) {
       if (TG * g + jj >= nw) break;
 #pragma unroll
-      for (int mt = 0; mt < 4; ++mt)
+      for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int i = 0; i < 4; i += 2) {
           const uint32_t t = tvp[mt * 8 + jj * 2 + i / 2];
@@ -902,7 +907,28 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         }
     }
   }
-  finish_tile(a, logit, s_part, lane, wid, b, h, s0);
+  finish_tile<MT>(a, logit, s_part, lane, wid, b, h, s0);
+}
+
+template <int D, int NIN, int MT>
+void launch_packed_at(const GateArgs& a, const u32x4_t* pk, int precision, hipStream_t st) {
+  const dim3 grid((a.S + 16 * MT - 1) / (16 * MT), a.B * a.H);
+  if (precision == 0) hipLaunchKernelGGL((gate_bf16_kernel<D, NIN, 0, MT>), grid, dim3(kThreads), 0, st, a, pk);
+  else if (precision == 1) hipLaunchKernelGGL((gate_bf16p_kernel<D, NIN, 1, MT>), grid, dim3(kThreads), 0, st, a, pk);
+  else hipLaunchKernelGGL((gate_bf16p_kernel<D, NIN, 2, MT>), grid, dim3(kThreads), 0, st, a, pk);
+}
+
+template <int MT>
+void launch_packed(const GateArgs& a, const u32x4_t* pk, int n_in, int precision, hipStream_t st) {
+  if (a.D == 128) {
+    if (n_in == 1) launch_packed_at<128, 1, MT>(a, pk, precision, st);
+    else if (n_in == 2) launch_packed_at<128, 2, MT>(a, pk, precision, st);
+    else launch_packed_at<128, 3, MT>(a, pk, precision, st);
+  } else {
+    if (n_in == 1) launch_packed_at<64, 1, MT>(a, pk, precision, st);
+    else if (n_in == 2) launch_packed_at<64, 2, MT>(a, pk, precision, st);
+    else launch_packed_at<64, 3, MT>(a, pk, precision, st);
+  }
 }
 
 template <int K>
@@ -1020,23 +1046,17 @@ extern "C" int wgkv_gate_scores(
     }
     if (aligned) {
       const u32x4_t* pk = (const u32x4_t*)w1_packed;
-      const dim3 grid((seq_len + kTok - 1) / kTok, batch * num_kv_heads);
-#define WGKV_GATE_BF16(DD, NN)                                                                              \
-  do {                                                                                                      \
-    if (precision == 0) hipLaunchKernelGGL((gate_bf16_kernel<DD, NN, 0>), grid, dim3(kThreads), 0, st, a, pk); \
-    else if (precision == 1) hipLaunchKernelGGL((gate_bf16p_kernel<DD, NN, 1>), grid, dim3(kThreads), 0, st, a, pk); \
-    else hipLaunchKernelGGL((gate_bf16p_kernel<DD, NN, 2>), grid, dim3(kThreads), 0, st, a, pk);             \
-  } while (0)
-      if (head_dim == 128) {
-        if (n_in == 1) WGKV_GATE_BF16(128, 1);
-        else if (n_in == 2) WGKV_GATE_BF16(128, 2);
-        else WGKV_GATE_BF16(128, 3);
-      } else {
-        if (n_in == 1) WGKV_GATE_BF16(64, 1);
-        else if (n_in == 2) WGKV_GATE_BF16(64, 2);
-        else WGKV_GATE_BF16(64, 3);
-      }
-#undef WGKV_GATE_BF16
+      // Tokens per workgroup: 64, or 32 while the 64-token workgroups would not
+      // outnumber the CUs.  A launch then takes as long as one workgroup, whose
+      // time is its epilogue's activations and products: half as many take
+      // two thirds of the time.  Above, a second workgroup per CU hides them
+      // and the weights, read once per workgroup, count.  8 heads of D 128,
+      // inner 512, 64 / 32 tokens: fp32 parameters 500 tokens 26.2 / 17.1 us,
+      // 1024 26.7 / 18.4, 2048 28.1 / 25.4, 3000 34.4 / 38.8, 4096 35.9 / 46.1;
+      // bf16 parameters 12.0 / 8.4, 13.2 / 9.7, 14.1 / 12.2, 18.1 / 18.1, 18.9 /
+      // 21.7.  A token's arithmetic is the same in both.
+      if ((int64_t)((seq_len + 63) / 64) * batch * num_kv_heads <= cu_count()) launch_packed<2>(a, pk, n_in, precision, st);
+      else launch_packed<4>(a, pk, n_in, precision, st);
       return hipGetLastError() == hipSuccess ? WGKV_OK : WGKV_ERR_HIP;
     }
   }

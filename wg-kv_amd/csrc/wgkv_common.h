@@ -213,6 +213,19 @@ WGKV_DEVICE void copy_rows1(const uint16_t* a, int64_t ss, int n, int D, Src src
   }
 }
 
+// Compute units of the current device (256 where it cannot be asked).
+inline int cu_count() {
+  static int cached[64] = {0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (cached[dev] == 0) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    cached[dev] = n;
+  }
+  return cached[dev];
+}
+
 #define WGKV_HIP_CHECK(expr)                       \
   do {                                             \
     hipError_t _e = (expr);                        \
