@@ -161,21 +161,33 @@ __device__ __forceinline__ uint32_t fkey(float f) {
   return u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);
 }
 
+// Largest / smallest of x over the wave (DPP within rows of 16, then scalar).
+__device__ __forceinline__ uint32_t wave_umax(uint32_t x) {
+  x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, WGKV_DPP_QP_1032, 0xf, 0xf, false));
+  x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, WGKV_DPP_QP_2301, 0xf, 0xf, false));
+  x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, WGKV_DPP_ROW_HALF_MIRROR, 0xf, 0xf, false));
+  x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, WGKV_DPP_ROW_MIRROR, 0xf, 0xf, false));
+  const uint32_t a = max((uint32_t)__builtin_amdgcn_readlane((int)x, 0), (uint32_t)__builtin_amdgcn_readlane((int)x, 16));
+  const uint32_t b = max((uint32_t)__builtin_amdgcn_readlane((int)x, 32), (uint32_t)__builtin_amdgcn_readlane((int)x, 48));
+  return max(a, b);
+}
+
 // The selection of a head's `keep` largest of `full` page scores (0 < keep <
 // full) by one workgroup, kept pages written in page order from out on.  The
 // keep-th largest key T is found two bits at a time -- the largest T with at
 // least `keep` keys >= T -- with counts from ballots: no histogram, whose
-// bins the equal exponents of page scores crowd into.  Scores rounded to bf16
-// differ only in the key's upper half: 8 steps instead of 16.  With STAGED
-// the keys are read once and kept in LDS (heads of up to kMaxKeys pages),
-// else the scores are read again in every step.
+// bins the equal exponents of page scores crowd into.  The bits that all keys
+// share (their exponents, mostly) need no step, and scores rounded to bf16
+// differ only in the key's upper half: 4 or 5 steps of ~1100 cycles instead
+// of 16.  With STAGED the keys are read once and kept in LDS (heads of up to
+// kMaxKeys pages), else the scores are read again in every step.
 constexpr int kMaxKeys = 12288;  // a multiple of 8 * kThreads
 constexpr int kWaves = kThreads / 64;
-constexpr int kRowGroup = 64;  // rows of kThreads pages placed per scan
+constexpr int kRows = 8;  // rows of kThreads pages handled together
 
 template <bool BF16, bool STAGED>
 __device__ void select_pages(const float* sc, int full, int keep, const int32_t* pages, int32_t* out,
-                             uint32_t* s_key, int (*s_cnt)[3][kWaves], int* s_pref, int* s_tmp) {
+                             uint32_t* s_key, int (*s_cnt)[3][kWaves], int* s_pref) {
   constexpr int BITS = BF16 ? 16 : 32;
   const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
   const int rows = (full + kThreads - 1) / kThreads;  // of kThreads pages
@@ -185,29 +197,49 @@ __device__ void select_pages(const float* sc, int full, int keep, const int32_t*
     return p < full ? x : 0u;
   };
   auto key_at = [&](int p) { return STAGED ? s_key[p] : read_key(p); };
-  if (STAGED) {  // whole groups of eight rows; each thread reads back only its own keys: no barrier
-    for (int r0 = 0; r0 < rows; r0 += 8) {
-      uint32_t x[8];
+  // whole groups of rows; each thread reads back only its own keys: no barrier
+  uint32_t hi = 0, lo = 0;  // the largest key, and the largest complement of one
+  for (int r0 = 0; r0 < rows; r0 += kRows) {
+    uint32_t x[kRows];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) x[j] = read_key((r0 + j) * kThreads + t);
+    for (int j = 0; j < kRows; ++j) x[j] = read_key((r0 + j) * kThreads + t);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) s_key[(r0 + j) * kThreads + t] = x[j];
+    for (int j = 0; j < kRows; ++j) {
+      const int p = (r0 + j) * kThreads + t;
+      if (STAGED) s_key[p] = x[j];
+      hi = max(hi, x[j]);
+      lo = max(lo, p < full ? ~x[j] : 0u);
     }
   }
-  uint32_t T = 0;
+  hi = wave_umax(hi);
+  lo = wave_umax(lo);
+  if (lane == 0) {
+    s_pref[wid] = (int)hi;
+    s_pref[kWaves + wid] = (int)lo;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    hi = max(hi, (uint32_t)s_pref[w]);
+    lo = max(lo, (uint32_t)s_pref[kWaves + w]);
+  }
+  const uint32_t diff = hi ^ ~lo;  // the bits in which the largest and the smallest key differ
+  const int top = diff ? (33 - __builtin_clz(diff)) & ~1 : 0;  // an even number of low bits that holds them
+  uint32_t T = top < 32 ? hi >> top << top : 0u;
+  T = __builtin_amdgcn_readfirstlane(T);
   int above = 0;  // keys >= T's last tested successor: keys > T at the end
 #pragma unroll 1
-  for (int shift = BITS - 2, step = 0; shift >= 0; shift -= 2, step ^= 1) {
+  for (int shift = __builtin_amdgcn_readfirstlane(top) - 2, step = 0; shift >= 0; shift -= 2, step ^= 1) {
     int c[3] = {0, 0, 0};
 #pragma unroll 1
-    for (int r0 = 0; r0 < rows; r0 += 8) {
-      uint32_t x[8];
+    for (int r0 = 0; r0 < rows; r0 += kRows) {
+      uint32_t x[kRows];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) x[j] = key_at((r0 + j) * kThreads + t);
+      for (int j = 0; j < kRows; ++j) x[j] = key_at((r0 + j) * kThreads + t);
 #pragma unroll
       for (int d = 0; d < 3; ++d)
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
+        for (int j = 0; j < kRows; ++j)
           c[d] += __builtin_popcountll(__builtin_amdgcn_ballot_w64(x[j] >= (T | ((uint32_t)(d + 1) << shift))));
     }
     // a step's counts are read before the next step's barrier: two sets suffice
@@ -219,41 +251,41 @@ __device__ void select_pages(const float* sc, int full, int keep, const int32_t*
     for (int d = 0; d < 3; ++d)
       c[d] = (s_cnt[step][d][0] + s_cnt[step][d][1]) + (s_cnt[step][d][2] + s_cnt[step][d][3]);
     const int digit = c[2] >= keep ? 3 : c[1] >= keep ? 2 : c[0] >= keep ? 1 : 0;
-    T |= (uint32_t)digit << shift;
+    T = __builtin_amdgcn_readfirstlane(T | (uint32_t)digit << shift);
     if (digit < 3) above = c[digit];
   }
-  T = __builtin_amdgcn_readfirstlane(T);
   // kept: key > T, plus the first need_eq pages (in page order) with key ==
-  // T.  kRowGroup rows at a time: each (row, wave)'s two counts packed in one
-  // word, their prefix in page order, then the kept pages' places.
+  // T.  kRows rows at a time: each (row, wave)'s two counts packed in one word,
+  // their prefix in page order, then the kept pages' places; the page ids are
+  // requested first.
   const int need_eq = keep - above;
   int base_gt = 0, base_eq = 0;  // before the group (a group's own counts fit 16 bits)
-  for (int g0 = 0; g0 < rows; g0 += kRowGroup) {
-    const int gr = min(kRowGroup, rows - g0);
-    __syncthreads();
-    for (int r = 0; r < gr; ++r) {
-      const int p = (g0 + r) * kThreads + t;
+  for (int r0 = 0; r0 < rows; r0 += kRows) {
+    int32_t id[kRows];
+    uint64_t gt[kRows], eq[kRows];
+#pragma unroll
+    for (int j = 0; j < kRows; ++j) id[j] = pages[min((r0 + j) * kThreads + t, full - 1)];
+    __syncthreads();  // s_pref is free
+#pragma unroll
+    for (int j = 0; j < kRows; ++j) {
+      const int p = (r0 + j) * kThreads + t;
       const uint32_t x = key_at(p);
-      const int gt = __builtin_popcountll(__builtin_amdgcn_ballot_w64(x > T));
-      const int eq = __builtin_popcountll(__builtin_amdgcn_ballot_w64(x == T && p < full));
-      if (lane == 0) s_pref[r * kWaves + wid] = gt << 16 | eq;
+      gt[j] = __builtin_amdgcn_ballot_w64(x > T);
+      eq[j] = __builtin_amdgcn_ballot_w64(x == T && p < full);
+      if (lane == 0) s_pref[j * kWaves + wid] = __builtin_popcountll(gt[j]) << 16 | __builtin_popcountll(eq[j]);
     }
     __syncthreads();
-    int total = 0;
-    const int pref = block_exclusive_scan_256(t < gr * kWaves ? s_pref[t] : 0, s_tmp, &total);
-    s_pref[t] = pref;
-    __syncthreads();
-    for (int r = 0; r < gr; ++r) {
-      const int p = (g0 + r) * kThreads + t;
-      const uint32_t x = key_at(p);
-      const uint64_t gt = __builtin_amdgcn_ballot_w64(x > T);
-      const uint64_t eq = __builtin_amdgcn_ballot_w64(x == T && p < full);
-      const int before = s_pref[r * kWaves + wid];
-      const uint64_t below = (1ull << lane) - 1;
-      const int rank_gt = base_gt + (before >> 16) + __builtin_popcountll(gt & below);
-      const int rank_eq = base_eq + (before & 0xffff) + __builtin_popcountll(eq & below);
-      if ((gt >> lane & 1) || ((eq >> lane & 1) && rank_eq < need_eq)) out[rank_gt + min(rank_eq, need_eq)] = pages[p];
+    const int mine = lane < kRows * kWaves ? s_pref[lane] : 0;
+    const int incl = wave_incl_scan(mine, lane);
+    const uint64_t below = (1ull << lane) - 1;
+#pragma unroll
+    for (int j = 0; j < kRows; ++j) {
+      const int before = __builtin_amdgcn_readlane(incl - mine, __builtin_amdgcn_readfirstlane(j * kWaves + wid));
+      const int rank_gt = base_gt + (before >> 16) + __builtin_popcountll(gt[j] & below);
+      const int rank_eq = base_eq + (before & 0xffff) + __builtin_popcountll(eq[j] & below);
+      if ((gt[j] >> lane & 1) || ((eq[j] >> lane & 1) && rank_eq < need_eq)) out[rank_gt + min(rank_eq, need_eq)] = id[j];
     }
+    const int total = __builtin_amdgcn_readlane(incl, 63);
     base_gt += total >> 16;
     base_eq += total & 0xffff;
   }
@@ -262,14 +294,13 @@ __device__ void select_pages(const float* sc, int full, int keep, const int32_t*
 // One workgroup per head.  Bound by latency (a few memory round trips and the
 // steps' barriers); four waves rather than sixteen, whose barriers and scalar
 // counting cost more than the keys.  1638 pages per head, 8 heads: 15.0 us
-// with four LDS-histogram passes over the scores in memory, 10.4 us in this
+// with four LDS-histogram passes over the scores in memory, 8.1 us in this
 // form.
 template <bool BF16>
 __global__ __launch_bounds__(kThreads) void quest_select_kernel(SelectArgs a) {
   __shared__ uint32_t s_key[kMaxKeys];
   __shared__ int s_cnt[2][3][kWaves];
-  __shared__ int s_pref[kRowGroup * kWaves];
-  __shared__ int s_tmp[kThreads];
+  __shared__ int s_pref[kRows * kWaves];
   const int h = blockIdx.x, t = threadIdx.x;
   const int32_t* bt = a.bt + (int64_t)h * a.max_pages;
   int32_t* out = a.sel_bt + (int64_t)h * a.sel_cap;
@@ -285,9 +316,9 @@ __global__ __launch_bounds__(kThreads) void quest_select_kernel(SelectArgs a) {
   const int keep = k <= 0 ? 0 : (all ? full : k);
   if (keep > 0 && !all) {
     if (full <= kMaxKeys)
-      select_pages<BF16, true>(sc, full, keep, bt + a.lb, out + local_blocks, s_key, s_cnt, s_pref, s_tmp);
+      select_pages<BF16, true>(sc, full, keep, bt + a.lb, out + local_blocks, s_key, s_cnt, s_pref);
     else
-      select_pages<BF16, false>(sc, full, keep, bt + a.lb, out + local_blocks, s_key, s_cnt, s_pref, s_tmp);
+      select_pages<BF16, false>(sc, full, keep, bt + a.lb, out + local_blocks, s_key, s_cnt, s_pref);
   } else if (keep > 0) {
     for (int p = t; p < keep; p += kThreads) out[local_blocks + p] = bt[a.lb + p];
   }
