@@ -139,3 +139,20 @@ def test_ring_write_entry_points_argument_checks_without_gpu():
     assert rope(layer=4) == _lib.ERR_ARG
     assert rope(W=0) == _lib.ERR_ARG
     assert rope(pool=0x1002) == _lib.ERR_UNSUPPORTED  # ring rows are written 16 bytes at a time
+
+
+@pytest.mark.parametrize("head_dim", [0, -16])
+@pytest.mark.parametrize("norm", [False, True])
+def test_rope_rejects_an_empty_head_without_gpu(head_dim, norm):
+    """wgkv_rope_qkv and wgkv_rope_qkv_norm refuse a head_dim below 16 on the
+    host, before the launch's split divides by the threads of a head (the
+    fake pointers are never dereferenced)."""
+    from wgkv import _lib
+    L = _lib.lib()
+    f = 0x1000
+    t = (f, 0, 0, 0)  # a tensor and its strides
+    head = (*t, *t, *t, f, f, 0, 0, *t, *t, *t, 1, 1, 8, 2, head_dim)
+    if norm:
+        assert L.wgkv_rope_qkv_norm(*head, f, f, 1e-6, *t, None) == _lib.ERR_ARG
+    else:
+        assert L.wgkv_rope_qkv(*head, None) == _lib.ERR_ARG

@@ -544,7 +544,7 @@ int rope_launch(const void* q, int64_t q_sb, int64_t q_ss, int64_t q_sh,
                 int32_t head_dim, const void* q_norm_weight, const void* k_norm_weight, float eps,
                 void* k_pre, int64_t kp_sb, int64_t kp_ss, int64_t kp_sh, const RopeArgs& ring, void* stream) {
   if (!q || !k || !cos || !sin || !q_out || !k_out || (v == nullptr) != (v_out == nullptr)) return WGKV_ERR_ARG;
-  if (batch <= 0 || seq_len <= 0 || num_q_heads <= 0 || num_kv_heads <= 0) return WGKV_ERR_ARG;
+  if (batch <= 0 || seq_len <= 0 || num_q_heads <= 0 || num_kv_heads <= 0 || head_dim <= 0) return WGKV_ERR_ARG;
   if (head_dim % 16) return WGKV_ERR_UNSUPPORTED;
   if ((q_norm_weight || k_norm_weight) && head_dim > 256) return WGKV_ERR_UNSUPPORTED;
   if (misaligned(q_norm_weight) || misaligned(k_norm_weight) || misaligned(k_pre)) return WGKV_ERR_UNSUPPORTED;
