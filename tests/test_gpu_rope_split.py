@@ -37,6 +37,43 @@ def test_split_matches_torch(B, S, Hq, Hkv, D):
     same(vo, v)
 
 
+@pytest.mark.parametrize("S", [1, 37])
+@pytest.mark.parametrize("Hq,Hkv,D", [(1, 1, 48), (5, 2, 80), (8, 2, 96), (3, 3, 112), (2, 1, 176), (48, 8, 240),
+                                      (1, 1, 16), (8, 2, 32), (64, 8, 128), (64, 8, 256)])
+def test_head_norms_over_head_dims(Hq, Hkv, D, S):
+    """The per-head norm for every multiple of 16 up to 256, where the threads
+    of a head are a power of two and where they are not, one or several
+    workgroups per token.  The normalised k is within a bf16 step of the torch
+    norm (its sum of squares is summed in another order: relative 1.5 * 2^-7
+    with the weight's rounding) and rotates to exactly the rotated k; the
+    rotated q is within 2^-5 of its operands' magnitudes."""
+    from wgkv import model_ops
+    from wgkv.attention import apply_rotary_pos_emb
+    g = torch.Generator(device="cuda").manual_seed(Hq * D + S)
+    # heads of different magnitudes: a sum over another head's elements shows
+    buf = torch.randn(1, S, Hq + 2 * Hkv, D, generator=g, device="cuda")
+    buf = (buf * torch.exp(2 * torch.randn(1, S, Hq + 2 * Hkv, 1, generator=g, device="cuda"))).to(torch.bfloat16)
+    q, k, v = (t.transpose(1, 2) for t in (buf[:, :, :Hq], buf[:, :, Hq:Hq + Hkv], buf[:, :, Hq + Hkv:]))
+    ang = torch.rand(1, S, D, generator=g, device="cuda") * 6.28
+    cos, sin = ang.cos().to(torch.bfloat16), ang.sin().to(torch.bfloat16)
+    qw, kw = ((1 + 0.1 * torch.randn(D, generator=g, device="cuda")).to(torch.bfloat16) for _ in range(2))
+    print(f"[rope split] norms Hq{Hq} Hkv{Hkv} D{D} S{S}", flush=True)
+
+    def norm(x, w):
+        xf = x.float()
+        return w * (xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + 1e-6)).to(torch.bfloat16)
+
+    qo, ko, vo, kp = model_ops.rope_qkv(q, k, v, cos, sin, qw, kw, 1e-6)
+    qn, kn = norm(q, qw), norm(k, kw)
+    assert ((kp.float() - kn.float()).abs() <= 1.5 * 2 ** -7 * kn.float().abs()).all()
+    qr, kr = apply_rotary_pos_emb(qn, kp, cos, sin)
+    same(ko, kr)
+    same(vo, v)
+    mag = qn.float().abs()
+    mag = mag + torch.cat((mag[..., D // 2:], mag[..., :D // 2]), -1)
+    assert ((qo.float() - qr.float()).abs() <= 2 ** -5 * mag).all()
+
+
 def test_rounding_of_special_values():
     from wgkv import model_ops
     x = torch.tensor([float("inf"), float("-inf"), 1e-40, 3.3e38, -3.3e38, 0.0, -0.0, 1.0], device="cuda").to(torch.bfloat16)

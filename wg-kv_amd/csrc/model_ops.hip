@@ -141,8 +141,10 @@ __global__ __launch_bounds__(kNormThreads) void rms_norm_kernel(NormArgs a) {
 // v is copied, so the three outputs can share one buffer and strides.
 // Optionally q and k first get Qwen3's per-head RMSNorm (nw[0], nw[1]):
 // x <- bf16(w * bf16(x * rsqrt(mean_head(x^2) + eps))), the sum of squares
-// reduced over the D/16 threads of the head; the normalised k before the
-// rotation (the gate's pre-RoPE key) is also stored to kpre.
+// reduced over the D/16 threads of the head (padded to a power of two by
+// threads that add nothing, so that a head's threads are an aligned group of
+// lanes); the normalised k before the rotation (the gate's pre-RoPE key) is
+// also stored to kpre.
 constexpr int kRopeThreads = 512;  // at most; whole waves
 
 struct RopeArgs {
@@ -155,6 +157,7 @@ struct RopeArgs {
   const uint16_t* sin;
   int64_t cs_sb, cs_ss;
   int B, S, D;
+  int tph;       // threads per head: D / 16, with a norm the next power of two
   int wgs, tpw;  // workgroups per token, or tokens per workgroup (one of them is 1)
   const uint16_t* nw[2];
   float eps;
@@ -179,11 +182,15 @@ struct RopeArgs {
 // so a thread divides 32-bit indices only; with the hardware's bf16 conversions
 // the launch is bound by memory: 4096 tokens of 32 + 2 x 8 heads of 128 (100
 // MB) 28.0 us with 64-bit divisions and roundings in integer arithmetic, 19.7
-// us (5.1 TB/s) in this form.
+// us (5.1 TB/s) in this form.  PAD: heads padded to a power of two threads (a
+// norm over 48, 80, 96, ... values), an instance of its own because the
+// padding's early returns keep the cos / sin loads from going out with the
+// rows': 64 + 2 x 8 heads of 128 took 30.1 us instead of 28.1.
+template <bool PAD>
 __global__ __launch_bounds__(kRopeThreads) void rope_kernel(RopeArgs a) {
-  const int half = a.D / 2, hch = half / 8;
+  const int half = a.D / 2, tph = a.tph;
   const int Ht = a.H[0] + a.H[1] + a.H[2];
-  const unsigned items = Ht * hch;
+  const unsigned items = Ht * tph;
   int tok = blockIdx.x / a.wgs;
   unsigned idx = (blockIdx.x - tok * a.wgs) * blockDim.x + threadIdx.x;  // within the token
   if (a.tpw > 1) {
@@ -202,8 +209,9 @@ __global__ __launch_bounds__(kRopeThreads) void rope_kernel(RopeArgs a) {
     }
   }
   if (idx >= items) return;
-  int hh = (int)(idx / (unsigned)hch);
-  const int c = (int)idx - hh * hch;
+  int hh = (int)(idx / (unsigned)tph);
+  const int c = (int)idx - hh * tph;
+  const bool live = !PAD || c * 8 < half;  // else the head's padding
   const int b = tok / a.S, s = tok - b * a.S;
   int ten = 0;
   if (hh >= a.H[0]) {
@@ -216,11 +224,12 @@ __global__ __launch_bounds__(kRopeThreads) void rope_kernel(RopeArgs a) {
   }
   const uint16_t* src = a.in[ten] + b * a.is[ten][0] + s * a.is[ten][1] + hh * a.is[ten][2];
   uint16_t* dst = a.out[ten] + b * a.os[ten][0] + s * a.os[ten][1] + hh * a.os[ten][2];
-  const int d0 = c * 8;
+  const int d0 = live ? c * 8 : 0;
   const u32x4_t w1 = *(const u32x4_t*)(src + d0), w2 = *(const u32x4_t*)(src + half + d0);
   // this head's row of the ring (decode row: b = s = 0)
   const int64_t rrow = ((int64_t)hh * a.W + slot) * a.D;
   if (ten == 2) {
+    if (!live) return;
     *(u32x4_t*)(dst + d0) = w1;
     *(u32x4_t*)(dst + half + d0) = w2;
     if (a.ring) {
@@ -235,16 +244,18 @@ __global__ __launch_bounds__(kRopeThreads) void rope_kernel(RopeArgs a) {
   unpack8(w1, x1);
   unpack8(w2, x2);
   if (a.nw[ten]) {
-    // the head's D/16 threads are consecutive lanes (hch divides 64)
+    // the head's threads are tph <= 16 consecutive lanes, tph a power of two
     float ss = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) ss = fmaf(x1[e], x1[e], ss);
 #pragma unroll
     for (int e = 0; e < 8; ++e) ss = fmaf(x2[e], x2[e], ss);
-    if (hch >= 2) ss += dpp_f32<WGKV_DPP_QP_1032>(ss);
-    if (hch >= 4) ss += dpp_f32<WGKV_DPP_QP_2301>(ss);
-    if (hch >= 8) ss += dpp_f32<WGKV_DPP_ROW_HALF_MIRROR>(ss);
-    if (hch >= 16) ss += dpp_f32<WGKV_DPP_ROW_MIRROR>(ss);
+    ss = live ? ss : 0.f;
+    if (tph >= 2) ss += dpp_f32<WGKV_DPP_QP_1032>(ss);
+    if (tph >= 4) ss += dpp_f32<WGKV_DPP_QP_2301>(ss);
+    if (tph >= 8) ss += dpp_f32<WGKV_DPP_ROW_HALF_MIRROR>(ss);
+    if (tph >= 16) ss += dpp_f32<WGKV_DPP_ROW_MIRROR>(ss);
+    if (!live) return;
     const float scale = rsqrtf(ss / (float)a.D + a.eps);
     float n1[8], n2[8];
     unpack8(*(const u32x4_t*)(a.nw[ten] + d0), n1);
@@ -260,6 +271,7 @@ __global__ __launch_bounds__(kRopeThreads) void rope_kernel(RopeArgs a) {
       *(u32x4_t*)(kp + half + d0) = pack8(x2);
     }
   }
+  if (!live) return;
   if (ten == 1 && a.ring) {  // the pre-RoPE key (normalised when the head norm is on)
     *(u32x4_t*)(a.ring_pk + rrow + d0) = pack8(x1);
     *(u32x4_t*)(a.ring_pk + rrow + half + d0) = pack8(x2);
@@ -596,7 +608,10 @@ int rope_launch(const void* q, int64_t q_sb, int64_t q_ss, int64_t q_sh,
   a.W = ring.W;
   // a token's threads in as few workgroups of whole waves as hold them, or as
   // many tokens as 256 threads hold
-  const int items = (a.H[0] + a.H[1] + a.H[2]) * (head_dim / 16);
+  a.tph = head_dim / 16;
+  if (q_norm_weight || k_norm_weight)
+    while (a.tph & (a.tph - 1)) a.tph += a.tph & -a.tph;  // up to the next power of two
+  const int items = (a.H[0] + a.H[1] + a.H[2]) * a.tph;
   const int64_t tokens = (int64_t)batch * seq_len;
   if (tokens > INT32_MAX) return WGKV_ERR_UNSUPPORTED;
   a.wgs = (items + kRopeThreads - 1) / kRopeThreads;
@@ -604,7 +619,10 @@ int rope_launch(const void* q, int64_t q_sb, int64_t q_ss, int64_t q_sh,
   const int threads = (((items + a.wgs - 1) / a.wgs) * a.tpw + 63) / 64 * 64;
   const int64_t grid = (tokens + a.tpw - 1) / a.tpw * a.wgs;
   if (grid > INT32_MAX) return WGKV_ERR_UNSUPPORTED;
-  hipLaunchKernelGGL(rope_kernel, dim3((unsigned)grid), dim3(threads), 0, (hipStream_t)stream, a);
+  if (a.tph * 16 == head_dim)
+    hipLaunchKernelGGL(rope_kernel<false>, dim3((unsigned)grid), dim3(threads), 0, (hipStream_t)stream, a);
+  else
+    hipLaunchKernelGGL(rope_kernel<true>, dim3((unsigned)grid), dim3(threads), 0, (hipStream_t)stream, a);
   return hipGetLastError() == hipSuccess ? WGKV_OK : WGKV_ERR_HIP;
 }
 
