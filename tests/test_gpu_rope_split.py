@@ -74,6 +74,34 @@ def test_head_norms_over_head_dims(Hq, Hkv, D, S):
     assert ((qo.float() - qr.float()).abs() <= 2 ** -5 * mag).all()
 
 
+def test_more_threads_than_one_launch_holds():
+    """129 threads of each token in workgroups of 192: more than 2^32 threads
+    for 25 million tokens, so the call takes several launches.  Every token
+    reads the same rows (strides of 0) and writes its own k row."""
+    from wgkv import _lib
+    S, Hq, Hkv, D = 25_000_000, 41, 1, 48
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn(Hq + 2 * Hkv, D, generator=g, device="cuda").to(torch.bfloat16)
+    cos, sin = (torch.randn(D, generator=g, device="cuda").to(torch.bfloat16) for _ in range(2))
+    out = torch.zeros(Hq + 2 * Hkv, D, dtype=torch.bfloat16, device="cuda")
+    ko = torch.full((S, D), float("nan"), dtype=torch.bfloat16, device="cuda")
+    q, k, v, qo, vo = x[:Hq], x[Hq:Hq + 1], x[Hq + 1:], out[:Hq], out[Hq + 1:]
+    row = (0, 0, D)
+    print("[rope split] 25M tokens", flush=True)
+    st = _lib.lib().wgkv_rope_qkv(
+        q.data_ptr(), *row, k.data_ptr(), *row, v.data_ptr(), *row, cos.data_ptr(), sin.data_ptr(), 0, 0,
+        qo.data_ptr(), *row, ko.data_ptr(), 0, D, D, vo.data_ptr(), *row, 1, S, Hq, Hkv, D,
+        _lib.stream_handle(x.device))
+    torch.cuda.synchronize()
+    assert st == 0
+
+    def rot(t):
+        return t * cos + torch.cat((-t[..., D // 2:], t[..., :D // 2]), -1) * sin
+
+    assert torch.equal(qo, rot(q)) and torch.equal(vo, v)
+    assert torch.equal(ko[:1], rot(k)) and bool((ko == ko[:1]).all())
+
+
 def test_rounding_of_special_values():
     from wgkv import model_ops
     x = torch.tensor([float("inf"), float("-inf"), 1e-40, 3.3e38, -3.3e38, 0.0, -0.0, 1.0], device="cuda").to(torch.bfloat16)

@@ -159,6 +159,7 @@ struct RopeArgs {
   int B, S, D;
   int tph;       // threads per head: D / 16, with a norm the next power of two
   int wgs, tpw;  // workgroups per token, or tokens per workgroup (one of them is 1)
+  unsigned tok0;  // this launch's first token
   const uint16_t* nw[2];
   float eps;
   uint16_t* kpre;
@@ -191,18 +192,19 @@ __global__ __launch_bounds__(kRopeThreads) void rope_kernel(RopeArgs a) {
   const int half = a.D / 2, tph = a.tph;
   const int Ht = a.H[0] + a.H[1] + a.H[2];
   const unsigned items = Ht * tph;
-  int tok = blockIdx.x / a.wgs;
+  unsigned tok = blockIdx.x / a.wgs;
   unsigned idx = (blockIdx.x - tok * a.wgs) * blockDim.x + threadIdx.x;  // within the token
   if (a.tpw > 1) {
     const unsigned u = threadIdx.x / items;
-    tok = tok * a.tpw + (int)u;
-    idx = u < (unsigned)a.tpw && tok < a.B * a.S ? threadIdx.x - u * items : items;
+    tok = tok * a.tpw + u;
+    idx = u < (unsigned)a.tpw && a.tok0 + tok < (unsigned)(a.B * a.S) ? threadIdx.x - u * items : items;
   }
+  tok += a.tok0;
   int slot = 0;
   if (a.ring) {
     const int lp = a.ring[0], ll = max(a.ring[1], 0);
     slot = min(max(ll < a.W ? ll : lp, 0), a.W - 1);  // pointers out of range stay inside the ring
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {  // one token, one launch
       const int cur = ll < a.W ? ll + 1 : a.W;
       for (int h = 0; h < a.H[1]; ++h) a.seqlens[h] = cur + a.glen[h];
       a.ring[2] = slot;
@@ -212,7 +214,7 @@ __global__ __launch_bounds__(kRopeThreads) void rope_kernel(RopeArgs a) {
   int hh = (int)(idx / (unsigned)tph);
   const int c = (int)idx - hh * tph;
   const bool live = !PAD || c * 8 < half;  // else the head's padding
-  const int b = tok / a.S, s = tok - b * a.S;
+  const int b = (int)tok / a.S, s = (int)tok - b * a.S;
   int ten = 0;
   if (hh >= a.H[0]) {
     hh -= a.H[0];
@@ -617,12 +619,17 @@ int rope_launch(const void* q, int64_t q_sb, int64_t q_ss, int64_t q_sh,
   a.wgs = (items + kRopeThreads - 1) / kRopeThreads;
   a.tpw = items < 256 ? (int)(256 / items < tokens ? 256 / items : tokens) : 1;
   const int threads = (((items + a.wgs - 1) / a.wgs) * a.tpw + 63) / 64 * 64;
-  const int64_t grid = (tokens + a.tpw - 1) / a.tpw * a.wgs;
-  if (grid > INT32_MAX) return WGKV_ERR_UNSUPPORTED;
-  if (a.tph * 16 == head_dim)
-    hipLaunchKernelGGL(rope_kernel<false>, dim3((unsigned)grid), dim3(threads), 0, (hipStream_t)stream, a);
-  else
-    hipLaunchKernelGGL(rope_kernel<true>, dim3((unsigned)grid), dim3(threads), 0, (hipStream_t)stream, a);
+  // a launch holds less than 2^32 threads; padding to whole waves, a call may need more
+  const int64_t per_launch = (int64_t)(UINT32_MAX / threads / a.wgs) * a.tpw;  // tokens
+  for (int64_t t0 = 0; t0 < tokens; t0 += per_launch) {
+    const int64_t n = tokens - t0 < per_launch ? tokens - t0 : per_launch;
+    const dim3 grid((unsigned)((n + a.tpw - 1) / a.tpw * a.wgs));
+    a.tok0 = (unsigned)t0;
+    if (a.tph * 16 == head_dim)
+      hipLaunchKernelGGL(rope_kernel<false>, grid, dim3(threads), 0, (hipStream_t)stream, a);
+    else
+      hipLaunchKernelGGL(rope_kernel<true>, grid, dim3(threads), 0, (hipStream_t)stream, a);
+  }
   return hipGetLastError() == hipSuccess ? WGKV_OK : WGKV_ERR_HIP;
 }
 
