@@ -18,6 +18,10 @@ DEV = "cuda"
     (70, 64, 128, 64, (1024, 8192), 0.1),          # eight
     (2, 64, 64, 16, (640, 640), 0.0),
     (2, 64, 64, 16, (640, 640), 1.0),
+    (16, 64, 64, 16, (64, 64, 65), 0.5),           # 16 lanes count a head's flags
+    (40, 64, 64, 16, (64, 64, 65), 0.5),           # four
+    (130, 64, 64, 16, (64, 64, 65), 0.5),          # one
+    (300, 64, 64, 16, (128, 191), 0.3),            # one, two passes over the heads
 ])
 def test_chunks(H, D, W, P, chunks, frac):
     from wgkv import ops

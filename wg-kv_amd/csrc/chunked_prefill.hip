@@ -45,6 +45,7 @@ struct ChunkArgs {
   int32_t* column_count;  // (H, R_chunk)
   int r0, rchunk;         // first global row block of the chunk, row blocks in the chunk
   int span;               // 64-position steps per admission workgroup
+  int lph;                // lanes that count a head's flags: 64, 16, 4 or 1
   // workspace, written by stage 0 and read by stage 1
   int32_t* adm;           // (H) positions admitted by the chunk
   int32_t* gl_before;     // (H) global lengths before the chunk
@@ -56,7 +57,7 @@ constexpr int kMaxHeads = 1024;
 
 // Virtual sequence of a chunk: ring positions (c0 > 0 only) then the chunk.
 __host__ __device__ __forceinline__ int vlen(const ChunkArgs& a) { return (a.c0 > 0 ? a.W : 0) + a.C; }
-__device__ __forceinline__ int vring(const ChunkArgs& a) { return a.c0 > 0 ? a.W : 0; }
+__host__ __device__ __forceinline__ int vring(const ChunkArgs& a) { return a.c0 > 0 ? a.W : 0; }
 
 // Admitted flags of head h among the first n virtual positions, this thread's
 // share (t of nt threads).
@@ -69,7 +70,7 @@ __device__ __forceinline__ int vcount(const ChunkArgs& a, int h, int n, int t, i
 
 // Admission of one chunk in one launch (workgroup = `span` steps of 64
 // virtual positions of one head).  Every workgroup first counts the admitted
-// flags of every head (a wave per head) and makes the same plan from them --
+// flags of every head (lph lanes per head) and makes the same plan from them --
 // totals, capacity checks before any write, pages bump-allocated in head order
 // -- so no workgroup waits for another; then it compacts its own positions
 // into the head's pages (new pages are numbered arithmetically from the plan,
@@ -83,9 +84,12 @@ __device__ __forceinline__ int vcount(const ChunkArgs& a, int h, int n, int t, i
 // Bound by latency: the launch waits on memory about three times (flags and
 // lengths, the head's last page id, K/V rows).  64 positions per workgroup
 // give 512 workgroups for a 4096-token chunk of 8 heads, each copying its
-// ~13 rows in one batch of loads; 512 positions and one copy in flight per
-// thread took 17.4 us, with the counts added into LDS by every thread; this
-// takes 9.5 us.  span grows with heads x positions (wgkv_chunk_cache_update).
+// ~13 rows in one batch of loads.  Launched back to back, W 1024, a later
+// 4096-token chunk: 8 heads 8.0 us (512 positions and one copy in flight per
+// thread took 11.4, with the counts added into LDS by every thread), 32 heads
+// 16.5 (29.4), 64 heads 27.4 (62.9); 64 tokens, W 64: 8 heads 4.8 (5.8), 64
+// heads 4.9 (5.9).  span grows with heads x positions and lph falls with the
+// heads (both in wgkv_chunk_cache_update).
 __global__ __launch_bounds__(kThreads) void chunk_admit_kernel(ChunkArgs a) {
   __shared__ int s_tot[kMaxHeads];    // admitted positions of each head
   __shared__ int s_wave[kWaves];
@@ -109,9 +113,11 @@ __global__ __launch_bounds__(kThreads) void chunk_admit_kernel(ChunkArgs a) {
   const int open_page = gl0 % a.page ? bt[gl0 / a.page] : 0;  // the head's last page, partly filled
 
   // ---- admitted counts of every head, and of this head before v0 ----------
-  for (int hh = wid; hh < a.H; hh += kWaves) {
-    const int c = wave_sum_int(vcount(a, hh, n_adm, lane, 64));
-    if (lane == 0) s_tot[hh] = c;
+  const int lph = a.lph, sub = t & (lph - 1);
+  for (int h0 = 0; h0 < a.H; h0 += kThreads / lph) {
+    const int hh = h0 + t / lph;
+    const int c = group_sum_int(hh < a.H ? vcount(a, hh, n_adm, sub, lph) : 0, lph);
+    if (sub == 0 && hh < a.H) s_tot[hh] = c;
   }
   const int pre = wave_sum_int(v0 > 0 ? vcount(a, h, min(v0, n_adm), t, kThreads) : 0);
   if (lane == 0) s_wave[wid] = pre;
@@ -302,6 +308,20 @@ extern "C" int wgkv_chunk_cache_update(
   // every workgroup repeats would outweigh its own steps
   const int steps = (max(1, vlen(a) - local_window) + kBlk - 1) / kBlk;
   a.span = min(kMaxSpan, max(1, (int)((int64_t)steps * num_kv_heads / 1024)));
+  // Lanes per head for the counting: the number that takes the fewest memory
+  // round trips (count_flags has four 16-flag loads per lane in flight, and a
+  // pass counts kThreads / lph heads).  A wave for every head took 17.3 us
+  // instead of 4.9 for 64 heads of 64 tokens, 35.5 instead of 10.4 for 1000,
+  // 24.5 instead of 16.5 for 32 heads of 4096.
+  const int gr = vring(a) / 16, gc = (max(0, vlen(a) - local_window - vring(a)) + 15) / 16;
+  int64_t best = INT64_MAX;
+  for (int l = 64; l >= 1; l /= 4) {
+    const int64_t trips = (int64_t)((num_kv_heads * l + kThreads - 1) / kThreads) * ((gr + 4 * l - 1) / (4 * l) + (gc + 4 * l - 1) / (4 * l));
+    if (trips < best) {
+      best = trips;
+      a.lph = l;
+    }
+  }
   int32_t* ws = (int32_t*)workspace;
   a.adm = ws;
   a.gl_before = ws + num_kv_heads;

@@ -96,6 +96,23 @@ WGKV_DEVICE int wave_incl_scan(int v, int lane) {
   return v;
 }
 
+// Sum of an int over an aligned group of n lanes, n one of 1, 4, 16, 64 and
+// the same in the whole wave (every lane of the group gets the total).
+WGKV_DEVICE int group_sum_int(int x, int n) {
+  if (n >= 4) {
+    x += __builtin_amdgcn_update_dpp(0, x, WGKV_DPP_QP_1032, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, WGKV_DPP_QP_2301, 0xf, 0xf, false);
+  }
+  if (n >= 16) {
+    x += __builtin_amdgcn_update_dpp(0, x, WGKV_DPP_ROW_HALF_MIRROR, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, WGKV_DPP_ROW_MIRROR, 0xf, 0xf, false);
+  }
+  if (n == 64)
+    x = (__builtin_amdgcn_readlane(x, 0) + __builtin_amdgcn_readlane(x, 16)) +
+        (__builtin_amdgcn_readlane(x, 32) + __builtin_amdgcn_readlane(x, 48));
+  return x;
+}
+
 // Sum of an int over all 64 lanes (every lane gets the total).
 WGKV_DEVICE int wave_sum_int(int x) {
 #pragma unroll
@@ -127,7 +144,7 @@ WGKV_DEVICE int block_exclusive_scan_256(int v, int* s_tmp /* >= 4 ints */, int*
   return before + incl - v;
 }
 
-// This thread's share (t of n threads, n >= 16) of the nonzero flags in
+// This thread's share (t of n threads) of the nonzero flags in
 // m[lo, hi): whole 16-byte groups as vectors, the ends -- rows of odd length
 // start anywhere -- as bytes.
 WGKV_DEVICE int count_flags(const uint8_t* m, int lo, int hi, int t, int n) {
@@ -137,8 +154,8 @@ WGKV_DEVICE int count_flags(const uint8_t* m, int lo, int hi, int t, int n) {
   const int groups = (hi - lo - head) >> 4;
   const int tail = hi - lo - head - groups * 16;
   int c = 0;
-  if (t < head) c += p[t] != 0;
-  if (t < tail) c += m[hi - tail + t] != 0;
+  for (int i = t; i < head; i += n) c += p[i] != 0;
+  for (int i = t; i < tail; i += n) c += m[hi - tail + i] != 0;
   const u32x4_t* v = (const u32x4_t*)(p + head);
   constexpr int U = 4;  // loads in flight
   for (int g0 = t; g0 < groups; g0 += n * U) {
