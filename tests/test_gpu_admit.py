@@ -56,6 +56,14 @@ def test_counting_in_the_plan_and_before_it(H, S):
     run_case(H, S, 64, 64, 16, 0.2, 3, seed=H)
 
 
+@pytest.mark.parametrize("H,S", [(5, 8192), (5, 8193), (70, 130), (130, 65), (200, 2049), (1024, 66)])
+def test_threads_per_head_in_the_plan(H, S):
+    """Up to four count tiles per head (8192 tokens) and above, and from 5 to
+    1024 heads: the plan's threads per head change with the tiles, its passes
+    over the heads with their number."""
+    run_case(H, S, 16, 16, 16, 0.3, 2, seed=H + S)
+
+
 @pytest.mark.parametrize("frac", [0.0, 1.0])
 def test_none_and_all_admitted(frac):
     run_case(2, 3000, 64, 128, 16, frac, 1, seed=7, defer=False)

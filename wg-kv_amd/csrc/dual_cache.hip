@@ -28,6 +28,7 @@ constexpr int kPlanWaves = kPlanThreads / 64;
 // tiles) 10.8 / 11.6 us, 6100 (24) 12.8 / 12.8, 9001 (40) 15.3 / 13.9, 32768
 // (128) 28.1 / 21.6.
 constexpr int kPlanCounts = 24;
+constexpr int kFewTiles = 4;  // count tiles per head that the plan takes with a thread per head
 
 struct AdmitArgs {
   const uint16_t* key;
@@ -70,10 +71,13 @@ __global__ __launch_bounds__(kThreads) void admit_count_kernel(AdmitArgs a) {
 // One workgroup: per-head totals (with COUNT from the flags themselves),
 // capacity checks, page allocation in head order
 // (src/modeling_layers.py:1303-1331), block-table rows, lengths.  A wave
-// counts a tile in two 16-byte loads per lane and takes a head's tiles in one
-// scan of 64, so the launch waits on memory a few times whatever the prompt's
-// length (one thread per head walking its tiles and pages took a memory round
-// trip for each).
+// counts a tile in two 16-byte loads per lane and takes a long prompt's head in
+// one scan of 64 tiles, so the launch waits on memory a few times whatever the
+// prompt's length (one thread per head walking its tiles and pages took a
+// memory round trip for each).  Heads of few tiles take a thread each, as a
+// wave each would go over many heads one after another: whole call, 130
+// tokens, 64 heads 14.4 us with a wave per head, 11.5 in this form, 128 heads
+// 18.1 / 12.5, 8 heads 10.8 / 10.4.
 template <bool COUNT>
 __global__ __launch_bounds__(kPlanThreads) void admit_plan_kernel(AdmitArgs a) {
   __shared__ int s_cnt[COUNT ? kPlanCounts : 1];
@@ -107,7 +111,25 @@ __global__ __launch_bounds__(kPlanThreads) void admit_plan_kernel(AdmitArgs a) {
     }
     __syncthreads();
   }
-  for (int h = wid; h < a.H; h += kPlanWaves) {
+  // few tiles: a thread per head, whose loads go out together; else a wave
+  const bool few = a.ntiles <= kFewTiles;
+  for (int h = few ? t : a.H; h < a.H; h += kPlanThreads) {
+    int c[kFewTiles];
+#pragma unroll
+    for (int tl = 0; tl < kFewTiles; ++tl) {
+      const int i = h * a.ntiles + min(tl, a.ntiles - 1);
+      c[tl] = COUNT ? s_cnt[i] : a.tile_cnt[i];
+    }
+    int run = 0;
+#pragma unroll
+    for (int tl = 0; tl < kFewTiles; ++tl)
+      if (tl < a.ntiles) {
+        a.tile_base[h * a.ntiles + tl] = run;
+        run += c[tl];
+      }
+    s_n[h] = run;
+  }
+  for (int h = few ? a.H : wid; h < a.H; h += kPlanWaves) {
     int run = 0;
     for (int t0 = 0; t0 < a.ntiles; t0 += 64) {
       const int tl = t0 + lane;
@@ -120,7 +142,8 @@ __global__ __launch_bounds__(kPlanThreads) void admit_plan_kernel(AdmitArgs a) {
     if (lane == 0) s_n[h] = run;
   }
   __syncthreads();
-  // first page of each head, relative to the bump pointer, and the checks
+  // first page of each head, relative to the bump pointer, and the checks (one
+  // wave: a scan over the whole workgroup costs 0.3 us at 8 heads)
   if (wid == 0) {
     int carry = 0, bad = 0;
     for (int h0 = 0; h0 < a.H; h0 += 64) {
@@ -147,15 +170,16 @@ __global__ __launch_bounds__(kPlanThreads) void admit_plan_kernel(AdmitArgs a) {
     return;
   }
   const int nf = s_nf;
-  for (int h = wid; h < a.H; h += kPlanWaves) {
+  const int g = few ? 16 : 64, sub = t & (g - 1);  // threads that write a head's rows
+  for (int h = t / g; h < a.H; h += kPlanThreads / g) {
     const int n = s_n[h], first = nf + s_pg[h];
-    if (lane == 0) {
+    if (sub == 0) {
       a.head_row[h] = (int64_t)first * a.page;
       if (n > 0) a.global_lengths[a.layer * a.H + h] = n;
     }
     const int pages = (n + a.page - 1) / a.page;
     int32_t* row = a.block_table + ((int64_t)a.layer * a.H + h) * a.max_pages + lb;
-    for (int i = lane; i < pages; i += 64) row[i] = first + i;
+    for (int i = sub; i < pages; i += g) row[i] = first + i;
   }
   if (t == 0) {
     *a.next_free = nf + s_total;
