@@ -76,3 +76,21 @@ def test_tile_edges_and_unaligned_rows(S):
     for h in range(H):
         n = int(ref[2][0, h].max(initial=0))
         assert np.array_equal(got[3][0, h, 0, :n], ref[3][0, h, 0, :n])
+
+
+@pytest.mark.parametrize("S", [2097152, 2097153, 2097217, 4194305, 6400001])
+def test_several_tiles_per_workgroup(S):
+    """Prompts of more than 512 tiles of 4096 positions, where a workgroup takes
+    two, three or four of them; the last workgroup full or not, and the total
+    of the listed positions with it."""
+    import wgkv
+    rng = np.random.default_rng(S)
+    mask = (rng.random((1, 2, S)) < 0.2)
+    md = wgkv.generate_sparse_indices(torch.from_numpy(mask).cuda(), 1024, 1, 2, S, exact_width=True)
+    n_list = (S - 1) // 64 * 64 + 1
+    start = np.maximum(0, np.arange((S + 63) // 64) * 64 - 1024 + 1)  # of each row block's band
+    for h in range(2):
+        pos = np.flatnonzero(mask[0, h, :n_list])
+        assert np.array_equal(md[2][0, h].cpu().numpy(), np.searchsorted(pos, start))
+        assert np.array_equal(md[3][0, h, 0, :pos.size].cpu().numpy(), pos)
+    assert md[3].shape[-1] == max(np.count_nonzero(mask[0, h, :n_list]) for h in range(2))
