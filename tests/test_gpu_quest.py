@@ -211,18 +211,13 @@ def test_selection_matches_reference_golden(name):
     print(f"[quest golden] {name}: {len(sc['steps'])} steps, lengths exact, selections equal up to ties", flush=True)
 
 
-@pytest.mark.parametrize("scores_bf16", [False, True])
-@pytest.mark.parametrize("G,D", [(1, 128), (3, 64), (4, 128), (5, 8), (8, 256)])
-@pytest.mark.parametrize("budget", [64, 64 + 16, 64 + 16 * 40, 64 + 16 * 1500])
-def test_selection_exact_over_head_lengths(G, D, budget, scores_bf16):
-    """Heads from no page to more than the selection keeps in registers (8192
-    pages).  Queries and bounds are small integers, so every score is exact in
-    fp32 and ties are many: the selection must be the largest scores, equal
-    ones by page order, whole numbers bit for bit."""
+def check_exact_selection(fulls, G, D, budget, scores_bf16):
+    """Heads of `fulls` full pages.  Queries and bounds are small integers, so
+    every score is exact in fp32 and ties are many: the selection must be the
+    largest scores, equal ones by page order, whole numbers bit for bit."""
     import types
     from wgkv import ops
     W, P = 64, 16
-    fulls = [0, 1, 15, 16, 17, 63, 64, 65, 1023, 1024, 1025, 2049, 8192, 8193, 12000]
     lens = [f * P + (i % 3) * 5 for i, f in enumerate(fulls)]
     H, lb = len(fulls), W // P
     g = torch.Generator().manual_seed(G * D + budget)
@@ -257,3 +252,52 @@ def test_selection_exact_over_head_lengths(G, D, budget, scores_bf16):
                           table[0, h, lb + full:lb + full + (1 if have > 0 and rem else 0)]))
         assert int(sel_len[0, h]) == W + keep * P + (rem if have > 0 and rem else 0), h
         assert torch.equal(sel_bt[0, h, :want.numel()].cpu(), want), h
+
+
+@pytest.mark.parametrize("scores_bf16", [False, True])
+@pytest.mark.parametrize("G,D", [(1, 128), (3, 64), (4, 128), (5, 8), (8, 256)])
+@pytest.mark.parametrize("budget", [64, 64 + 16, 64 + 16 * 40, 64 + 16 * 1500])
+def test_selection_exact_over_head_lengths(G, D, budget, scores_bf16):
+    """Heads from no page to nearly as many as the selection keeps in LDS
+    (12288 pages)."""
+    check_exact_selection([0, 1, 15, 16, 17, 63, 64, 65, 1023, 1024, 1025, 2049, 8192, 8193, 12000], G, D, budget,
+                          scores_bf16)
+
+
+@pytest.mark.parametrize("scores_bf16", [False, True])
+@pytest.mark.parametrize("G,D", [(1, 128), (4, 64)])
+@pytest.mark.parametrize("pages", [1, 2, 3, 64, 159, 160, 161, 255, 256, 257, 6000, 12287, 12288, 12289, 19999])
+def test_selection_exact_at_the_edges_of_its_forms(G, D, pages, scores_bf16):
+    """Heads ranked page by page (up to 160 or 256 pages), with the keys in LDS
+    (up to 12288) and with the scores read again in every step, the budget
+    from one page to all but one of each of them."""
+    check_exact_selection([2, 3, 65, 159, 160, 161, 255, 256, 257, 258, 12287, 12288, 12289, 20000], G, D,
+                          64 + 16 * pages, scores_bf16)
+
+
+@pytest.mark.parametrize("full,keep", [(f, k) for f in (100, 160, 161, 256, 257, 1000, 12289)
+                                       for k in (1, 7, 99, 254) if k < f])
+def test_selection_of_distinct_fp32_scores(full, keep):
+    """fp32 scores of both signs without ties, where the steps stop early: the
+    same pages as the reference's top-k of those scores in 64 bits."""
+    import types
+    from wgkv import ops
+    W, P, D = 64, 16, 8
+    lb = W // P
+    g = torch.Generator().manual_seed(full + keep)
+    # score of page i: q = (1, 2^-8, 0...) on bounds (a_i, b_i) -> distinct for distinct pairs of bf16 integers
+    v = torch.randperm(65536, generator=g)[:full] - 32768
+    lo = torch.zeros(lb + full, D)
+    lo[lb:, 0], lo[lb:, 1] = (v >> 8).float(), (v & 255).float()
+    q = torch.zeros(1, D)
+    q[0, 0], q[0, 1] = 1.0, 2.0 ** -8
+    bf = torch.bfloat16
+    table = torch.arange(lb + full, dtype=torch.int32).view(1, 1, -1)
+    c = types.SimpleNamespace(num_layers=1, num_kv_heads=1, head_dim=D, block_size=P, local_window_size=W,
+                              block_table=table.to(DEV), global_lengths=torch.tensor([[full * P]], dtype=torch.int32).to(DEV),
+                              quest_block_key_min=lo.to(bf).to(DEV), quest_block_key_max=lo.to(bf).to(DEV))
+    print(f"[quest] distinct full{full} keep{keep}", flush=True)
+    sel_len, sel_bt = ops.quest_select(c, 0, q.to(bf).to(DEV), W, W + P * keep, scores_bf16=False)
+    want = torch.topk(v.double(), keep).indices.sort().values + lb
+    assert int(sel_len[0, 0]) == W + keep * P
+    assert torch.equal(sel_bt[0, 0, lb:lb + keep].cpu().long(), want)

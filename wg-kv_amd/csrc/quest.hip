@@ -73,7 +73,7 @@ struct SelectArgs {
   const int32_t* len;  // global_lengths + layer * H
   const uint16_t* kmin;
   const uint16_t* kmax;
-  int H, G, D, page, local_tokens, scores_bf16;
+  int H, D, page, local_tokens, scores_bf16;
   int local_blocks, budget_blocks;  // pages of the local tokens and of the budget past them
   int32_t* sel_bt;     // (H, sel_cap)
   int sel_cap;
@@ -82,9 +82,9 @@ struct SelectArgs {
 };
 
 // Page scores: 16 lanes per page, 8 d-values each (16-byte loads of the
-// bounds; the queries' 8 values per group member held in registers), summed
-// per lane in d order and then over the 16 lanes; workgroups stride over the
-// head's full pages, two of them per lane group in flight.  Bound by latency
+// bounds and, from LDS, of the group members' queries), summed per lane in d
+// order and then over the 16 lanes; workgroups stride over the head's full
+// pages, two of them per lane group in flight.  Bound by latency
 // (a 128K prompt's 13.1K pages are 6.7 MB of bounds): the group size is a
 // template argument, as a runtime bound put the per-member sums in scratch
 // memory and read the queries from LDS value by value (30 us; now 6.2 us).
@@ -176,11 +176,17 @@ __device__ __forceinline__ uint32_t wave_umax(uint32_t x) {
 // full) by one workgroup, kept pages written in page order from out on.  The
 // keep-th largest key T is found two bits at a time -- the largest T with at
 // least `keep` keys >= T -- with counts from ballots: no histogram, whose
-// bins the equal exponents of page scores crowd into.  The bits that all keys
-// share (their exponents, mostly) need no step, and scores rounded to bf16
-// differ only in the key's upper half: 4 or 5 steps of ~1100 cycles instead
-// of 16.  With STAGED the keys are read once and kept in LDS (heads of up to
-// kMaxKeys pages), else the scores are read again in every step.
+// bins the equal exponents of page scores crowd into.  A step takes ~1100
+// cycles.  The leading bits that all keys share need no step, so scores of one
+// sign leave the exponent's out and scores of both signs leave out none.
+// Scores rounded to bf16 differ only in the key's upper half: at most 8 steps,
+// 4 or 5 where the scores have one sign.  fp32 scores would take up to 16, but
+// rarely tie: they stop once exactly `keep` keys reach T, after some log2(full)
+// bits below the shared ones (8 heads of 1638 pages, G 4, scores and selection
+// 15.2 us with all steps, 13.0 with the stop; with bf16 scores, which tie, the
+// test costs 0.3 of 12.6 us and is left out).  With STAGED the keys are read
+// once and kept in LDS (heads of up to kMaxKeys pages), else the scores are
+// read again in every step.
 constexpr int kMaxKeys = 12288;  // a multiple of 8 * kThreads
 constexpr int kWaves = kThreads / 64;
 constexpr int kRows = 8;  // rows of kThreads pages handled together
@@ -253,6 +259,14 @@ __device__ void select_pages(const float* sc, int full, int keep, const int32_t*
     const int digit = c[2] >= keep ? 3 : c[1] >= keep ? 2 : c[0] >= keep ? 1 : 0;
     T = __builtin_amdgcn_readfirstlane(T | (uint32_t)digit << shift);
     if (digit < 3) above = c[digit];
+    if constexpr (!BF16) {
+      const int reached = digit == 3 ? c[2] : digit == 2 ? c[1] : c[0];  // keys >= the new T (digit > 0)
+      if (digit > 0 && reached == keep) {  // exactly the kept keys: no lower bit matters
+        --T;
+        above = keep;
+        break;
+      }
+    }
   }
   // kept: key > T, plus the first need_eq pages (in page order) with key ==
   // T.  kRows rows at a time: each (row, wave)'s two counts packed in one word,
@@ -291,6 +305,38 @@ __device__ void select_pages(const float* sc, int full, int keep, const int32_t*
   }
 }
 
+// The same for a head of at most kThreads pages, a page per thread: a page is
+// kept if fewer than `keep` pages rank before it (a larger key, or the same
+// key and an earlier page).  One pass over the keys takes less than the steps
+// above for few pages (kFewPages, kFewPagesBf16): scores and selection of 8
+// heads, G 4, steps / this: fp32 scores of 100 pages 10.4 / 7.7 us, of 200
+// 10.5 / 10.0; bf16 scores of 60 pages 9.9 / 7.3, of 100 9.9 / 8.1, of 200
+// 10.0 / 10.3.
+constexpr int kFewPages = kThreads, kFewPagesBf16 = 160;
+
+__device__ void select_few_pages(const float* sc, int full, int keep, const int32_t* pages, int32_t* out,
+                                 uint32_t* s_key, int* s_pref) {
+  const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+  const int p = min(t, full - 1);
+  const int32_t id = pages[p];
+  const uint32_t x = fkey(sc[p]);
+  s_key[t] = t < full ? x : 0u;  // below every page's key
+  __syncthreads();
+  int rank = 0;
+  for (int q = 0; q < full; q += 4) {
+    const u32x4_t v = *(const u32x4_t*)(s_key + q);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) rank += v[e] > x || (v[e] == x && q + e < t);
+  }
+  const uint64_t kept = __builtin_amdgcn_ballot_w64(t < full && rank < keep);
+  if (lane == 0) s_pref[wid] = __builtin_popcountll(kept);
+  __syncthreads();
+  int at = __builtin_popcountll(kept & ((1ull << lane) - 1));
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) at += w < wid ? s_pref[w] : 0;
+  if (kept >> lane & 1) out[at] = id;
+}
+
 // One workgroup per head.  Bound by latency (a few memory round trips and the
 // steps' barriers); four waves rather than sixteen, whose barriers and scalar
 // counting cost more than the keys.  1638 pages per head, 8 heads: 15.0 us
@@ -298,7 +344,7 @@ __device__ void select_pages(const float* sc, int full, int keep, const int32_t*
 // form.
 template <bool BF16>
 __global__ __launch_bounds__(kThreads) void quest_select_kernel(SelectArgs a) {
-  __shared__ uint32_t s_key[kMaxKeys];
+  __shared__ __attribute__((aligned(16))) uint32_t s_key[kMaxKeys];
   __shared__ int s_cnt[2][3][kWaves];
   __shared__ int s_pref[kRows * kWaves];
   const int h = blockIdx.x, t = threadIdx.x;
@@ -315,7 +361,9 @@ __global__ __launch_bounds__(kThreads) void quest_select_kernel(SelectArgs a) {
   const bool all = k >= full;
   const int keep = k <= 0 ? 0 : (all ? full : k);
   if (keep > 0 && !all) {
-    if (full <= kMaxKeys)
+    if (full <= (BF16 ? kFewPagesBf16 : kFewPages))
+      select_few_pages(sc, full, keep, bt + a.lb, out + local_blocks, s_key, s_pref);
+    else if (full <= kMaxKeys)
       select_pages<BF16, true>(sc, full, keep, bt + a.lb, out + local_blocks, s_key, s_cnt, s_pref);
     else
       select_pages<BF16, false>(sc, full, keep, bt + a.lb, out + local_blocks, s_key, s_cnt, s_pref);
@@ -404,7 +452,6 @@ extern "C" int wgkv_quest_select(
   a.kmin = (const uint16_t*)key_min;
   a.kmax = (const uint16_t*)key_max;
   a.H = num_kv_heads;
-  a.G = G;
   a.D = head_dim;
   a.page = page_size;
   a.local_tokens = local_tokens;
