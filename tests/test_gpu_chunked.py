@@ -132,6 +132,16 @@ def test_chunked_equals_one_shot(L, H, G, D, W, chunks, frac, defer):
         assert torch.equal(got[l], ref[l]), (l, (got[l].float() - ref[l].float()).abs().max().item())
 
 
+@pytest.mark.parametrize("D,G,H,W,chunks", [(D, G, 8, 128, [128, 640, 1088, 133]) for D in (32, 64, 128) for G in (2, 4, 8)]
+                         + [(128, 4, 1, 128, [8192, 8192, 128]), (64, 4, 1, 128, [8192, 8192, 128])])
+def test_chunked_equals_one_shot_over_heads_per_workgroup(D, G, H, W, chunks):
+    """Chunks that take one, two and four query heads per workgroup: a short one
+    at the prompt's start, short ones later, one of more items than half the
+    CUs, and one whose last position lies beyond 16384, where D 128 stays at
+    four.  Outputs and caches equal the one-shot prompt's bit for bit."""
+    test_chunked_equals_one_shot(1, H, G, D, W, chunks, 0.3, False)
+
+
 @pytest.mark.parametrize("page", [32, 64])
 @pytest.mark.parametrize("L,H,G,D,W,chunks,frac,defer", [
     (2, 2, 4, 64, 256, [512, 320, 1024, 333], 0.4, False),

@@ -89,15 +89,11 @@ def test_long_prompt_sampled_rows(S, W, frac):
     assert err.max().item() <= 2e-2 and err.mean().item() <= 2e-3
 
 
-@pytest.mark.parametrize("D", [128, 64])
-def test_wide_kv_span_matches_contiguous(D):
-    """k/v whose rows span more than 2^31 bytes are loaded through the general
-    64-bit address path of the one-shot kernel; the same rows stored densely
-    take the 32-bit lane-offset path.  Both must give the same bits."""
+def check_wide_kv_span(B, Hkv, G, D):
     import wgkv
-    print(f"[prefill wide span] D{D}", flush=True)
+    print(f"[prefill wide span] B{B} G{G} D{D}", flush=True)
     dev = torch.device("cuda:0")
-    B, Hkv, G, S, W = 1, 2, 4, 2048, 256
+    S, W = 2048, 256
     q, k, v, gm = make(B, Hkv, G, S, D, 700, seed=97 + D)
     md = wgkv.generate_sparse_indices(gm.to(dev), W, B, Hkv, S)
     qd = q.to(dev).transpose(1, 2)
@@ -120,3 +116,40 @@ def test_wide_kv_span_matches_contiguous(D):
     ref64 = attention.masked_prefill(q, k, v, mask).float()
     err = (out.transpose(1, 2).float().cpu() - ref64).abs()
     assert err.max().item() <= 2e-2 and err.mean().item() <= 2e-3
+
+
+@pytest.mark.parametrize("D", [128, 64])
+def test_wide_kv_span_matches_contiguous(D):
+    """k/v whose rows span more than 2^31 bytes are loaded through the general
+    64-bit address path of the one-shot kernel; the same rows stored densely
+    take the 32-bit lane-offset path.  Both must give the same bits."""
+    check_wide_kv_span(1, 2, 4, D)
+
+
+@pytest.mark.parametrize("B,G,D", [(3, 4, 128), (1, 2, 128), (2, 4, 64), (3, 4, 64), (5, 2, 32), (1, 2, 32)])
+def test_wide_kv_span_over_heads_per_workgroup(B, G, D):
+    """The same with batches and groups that take four, two and one query heads
+    per workgroup (one above takes two at D 128 and one at D 64)."""
+    check_wide_kv_span(B, 2, G, D)
+
+
+@pytest.mark.parametrize("S", [200, 512, 513, 1024, 1025, 2100])
+@pytest.mark.parametrize("G", [2, 4, 8])
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_heads_per_workgroup(D, G, S):
+    """Both sides of every point at which a prompt of 8 KV heads goes over to
+    fewer query heads per workgroup: against the oracle on sampled rows, and
+    bit for bit against the same prompt in a batch of eight, which takes the
+    most heads a workgroup can (a query row's arithmetic does not depend on
+    the workgroup's other heads)."""
+    print(f"[prefill parity] heads per workgroup D{D} G{G} S{S}", flush=True)
+    W = 128
+    q, k, v, gm = make(1, 8, G, S, D, S // 5, seed=S + D + G)
+    out = run(q, k, v, gm, W)
+    g = torch.Generator().manual_seed(S)
+    rows = sorted(set([0, 63, 64, W, S - 1] + torch.randint(0, S, (3,), generator=g).tolist()))
+    err = (out[:, :, rows] - attention.sparse_prefill_rows(q, k, v, gm, W, rows).float()).abs()
+    assert err.max().item() <= 2e-2 and err.mean().item() <= 2e-3
+    batch = run(*(t.expand(8, *t.shape[1:]) for t in (q, k, v, gm)), W)
+    for b in range(8):
+        assert torch.equal(batch[b], out[0]), b

@@ -9,9 +9,10 @@
 // intersected with causality (key <= query).  Query head hq uses KV head
 // hq / G.
 //
-// Workgroup = (row block, b*Hkv + h), 2*G waves: wave w serves query head
-// h*G + w/2, rows (w%2)*32 .. +32 of the block, so each 64-key K/V tile is
-// staged in LDS once for all G heads.  Scores are computed transposed,
+// Work item = (row block, b*Hkv + h, group of HPW of the G query heads, HPW = 1,
+// 2 or 4: heads_per_wg), run by a workgroup of 2*HPW waves: wave w serves the
+// group's head w/2, rows (w%2)*32 .. +32 of the block, so each 64-key K/V tile
+// is staged in LDS once for HPW heads.  Scores are computed transposed,
 // S^T = K Q^T on v_mfma_f32_16x16x32_bf16 (K from LDS as the A operand, the
 // wave's queries held as the B operand), which leaves each lane with 4
 // consecutive keys of one query row: after the online softmax those
@@ -564,23 +565,41 @@ hipError_t launch(const PrefillArgs& a, hipStream_t st, bool chunked) {
 // Query heads per workgroup: the largest of 4, 2, 1 that divides G and lets
 // every wave load whole 1 KB blocks of a tile (2 * HPW waves, D / 8 blocks:
 // at most 2 heads at D = 32); G = 3 then takes one head per workgroup.  Halved
-// while the smaller workgroups would still get a CU each: a short prompt's
-// time is its longest item's, and a SIMD with one wave runs a tile sooner than
-// one that two waves share, which outweighs loading each K/V tile once per
-// half of the heads.  8 KV heads, G = 4, W 1024, 20 % admitted, 4 / 2 / 1
-// heads per workgroup: 500 tokens (64 items of 4 heads) 22.3 / 18.5 / 18.1 us,
-// 777 (104) 30.2 / 25.4 / 27.3, 1024 (128) 37.4 / 31.4 / 32.4, 2048 (256)
-// 48.3 / 64.4 / 65.8.
-int heads_per_wg(int head_dim, int G, int64_t rows) {
+// while the smaller workgroups would still get a CU each -- a short call's time
+// is its longest item's, and a SIMD with one wave runs a tile sooner than one
+// that two waves share -- unless the items are long: then loading a tile for
+// half of the heads costs more than the SIMD's second wave.  `reach` is the
+// last position, which bounds the tiles of an item; microseconds of 4 / 2 / 1
+// heads per workgroup, W 1024 and 20 % admitted unless said:
+//   4 to 2 heads at any length for D 64 (one-shot, 1 KV head, G 4, 8000 tokens
+//   51.2 / 48.1 / 50.0; a 1024-token chunk at 131072, 8 KV heads, G 4, W 128 499
+//   / 489 / 640) and up to kLongReach for D 128 (one-shot, 8 KV heads, G 4: 500
+//   tokens 22.6 / 18.9 / 18.5, 777 30.7 / 26.1 / 27.8, 1300 42.9 / 36.8 / 39.1,
+//   2048 49.4 / 65.6 / 68.3; 1 KV head, 8000 tokens 78.6 / 70.3 / 74.8, all
+//   admitted 217 / 199 / 213; a 128-token chunk of 8 KV heads, W 128, at 1024
+//   21.7 / 20.3 / 21.8, at 8192 60.3 / 59.9 / 66.2, at 16384 105 / 106 / 118, at
+//   131072 735 / 763 / 847);
+//   2 to 1 heads in the one-shot instance up to 512 positions for D 128 (G 2: 64
+//   tokens 8.0 (2) / 6.8, 500 18.5 / 18.0, 900 27.0 / 27.5, 8000 65.8 / 68.3), up
+//   to 2048 for D 64 (G 2: 900 20.2 / 20.2, 1500 26.0 / 25.4, 3000 with all
+//   admitted 55.3 / 57.1) and always for D 32 (16000 63.0 / 59.3), in the chunked
+//   instance up to 256 (D 128, G 2: 128 tokens at 0 10.0 / 9.2, at 512 16.8 /
+//   17.8, at 131072 768 / 855).
+constexpr int kLongReach = 16384;
+
+int heads_per_wg(int head_dim, int G, int64_t rows, int reach, bool chunked) {
   int h = head_dim == 32 ? 2 : 4;
   while (G % h) h >>= 1;
-  while (h > 1 && rows * (G / h) * 2 <= cu_count()) h >>= 1;
+  const auto halves_fit = [&] { return rows * (G / h) * 2 <= cu_count(); };
+  if (h == 4 && halves_fit() && (head_dim < 128 || reach <= kLongReach)) h = 2;
+  const int one = chunked ? 256 : head_dim == 128 ? 512 : head_dim == 64 ? 2048 : INT32_MAX;
+  if (h == 2 && halves_fit() && reach <= one) h = 1;
   return h;
 }
 
 hipError_t launch_any(PrefillArgs& a, hipStream_t st, int head_dim, int G, bool chunked) {
   a.G = G;
-  const int hpw = heads_per_wg(head_dim, G, (int64_t)a.R * a.B * a.Hkv);
+  const int hpw = heads_per_wg(head_dim, G, (int64_t)a.R * a.B * a.Hkv, a.S, chunked);
   if (head_dim == 128)
     return hpw == 1 ? launch<128, 1>(a, st, chunked) : hpw == 2 ? launch<128, 2>(a, st, chunked)
                     : launch<128, 4>(a, st, chunked);
