@@ -156,3 +156,16 @@ def test_rope_rejects_an_empty_head_without_gpu(head_dim, norm):
         assert L.wgkv_rope_qkv_norm(*head, f, f, 1e-6, *t, None) == _lib.ERR_ARG
     else:
         assert L.wgkv_rope_qkv(*head, None) == _lib.ERR_ARG
+
+
+def test_sparse_attn_func_refuses_an_empty_prompt(monkeypatch):
+    """No tokens: refused as metadata that does not match, not by a division by
+    its zero row blocks (the device check is passed by: nothing is launched)."""
+    import torch
+    from wgkv import ops
+    monkeypatch.setattr(ops, "_require_cuda", lambda *tensors: None)
+    q = torch.zeros(1, 0, 4, 64, dtype=torch.bfloat16)
+    k = torch.zeros(1, 0, 2, 64, dtype=torch.bfloat16)
+    none = torch.zeros(1, 2, 0, dtype=torch.int32)
+    with pytest.raises(AssertionError, match="metadata"):
+        ops.sparse_attn_func(q, k, k, none[:, 0], none[:, 0], none, none[:, :, None])

@@ -319,7 +319,7 @@ def sparse_attn_func(q, k, v, block_count, block_offset, column_count, column_in
     if qs[3] != 1 or ks[3] != 1:
         raise ValueError("head_dim must be contiguous")
     R = (S + 63) // 64
-    if block_count.numel() != R or block_offset.numel() % R or column_count.shape != (B, Hkv, R):
+    if R == 0 or block_count.numel() != R or block_offset.numel() % R or column_count.shape != (B, Hkv, R):
         raise AssertionError("metadata does not match (batch, heads, seq) with block 64")
     if softmax_scale is None:
         softmax_scale = D ** -0.5
