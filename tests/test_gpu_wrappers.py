@@ -89,3 +89,36 @@ def test_refused_stays_refused():
         wgkv.sparse_attn_func(q, k, k, md[0][..., :1], *md[1:])
     with pytest.raises(ValueError):
         wgkv.sparse_attn_func(q.cpu(), k, k, *md)
+
+
+@pytest.mark.parametrize("call", ["decode", "prefill"])
+def test_calls_run_on_the_current_stream(call):
+    """The handle is the current stream's, inside and outside a stream context,
+    and a call reads what work before it on that stream writes: the queries
+    arrive behind a long producer, so a launch on another stream reads zeros."""
+    import wgkv
+    from wgkv import _lib, ops, workloads
+    if call == "decode":
+        w = workloads.decode_ragged(ctx=3000, batch=3, window=256, seed=1)
+        args = [w.k_cache, w.v_cache, w.cache_seqlens, w.block_table.clamp(min=0), w.softmax_scale]
+        fn, q = ops.paged_decode_attn, w.q
+    else:
+        g = torch.Generator(device=DEV).manual_seed(5)
+        q, k, v = (torch.randn(1, 700, n, 64, generator=g, device=DEV).to(torch.bfloat16) for n in (8, 2, 2))
+        mask = torch.rand(1, 2, 700, generator=g, device=DEV) < 0.3
+        args = [k, v, *wgkv.generate_sparse_indices(mask, 128, 1, 2, 700)]
+        fn = wgkv.sparse_attn_func
+    ref = fn(q, *args)
+    late = torch.zeros_like(q)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    assert _lib.stream_handle(q.device) == torch.cuda.current_stream(q.device).cuda_stream
+    with torch.cuda.stream(side):
+        assert _lib.stream_handle(q.device) == side.cuda_stream == torch.cuda.current_stream(q.device).cuda_stream
+        torch.cuda._sleep(20_000_000)
+        late.copy_(q)
+        got = fn(late, *args)
+    assert not side.query()  # the call returned before the producer was done
+    assert _lib.stream_handle(q.device) == torch.cuda.current_stream(q.device).cuda_stream != side.cuda_stream
+    side.synchronize()
+    assert torch.equal(got, ref)
