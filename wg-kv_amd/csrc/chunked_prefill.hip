@@ -209,8 +209,8 @@ __global__ __launch_bounds__(kThreads) void chunk_admit_kernel(ChunkArgs a) {
 
 // After the chunk's attention: ring slot i <- chunk position C - W + i.
 // Grid (head, 64-slot group); a thread's rows are all requested before the
-// first store (one at a time: 9.2 us for 8 heads of W 1024 with the pre-RoPE
-// keys; 6.6 us).
+// first store (one at a time: 9.3 us for 8 heads of W 1024 with the pre-RoPE
+// keys, median of a trace; 6.7 us).
 __global__ __launch_bounds__(kThreads) void chunk_ring_kernel(ChunkArgs a) {
   if (*a.abort_flag) return;
   const int h = blockIdx.x;

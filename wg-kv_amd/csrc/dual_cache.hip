@@ -195,8 +195,8 @@ __global__ __launch_bounds__(kPlanThreads) void admit_plan_kernel(AdmitArgs a) {
 // ring's W rows are then copied by W/64 workgroups per head.  Bound by
 // latency: with 2048 positions per workgroup and one load per thread in
 // flight a single workgroup copied a head's whole ring, and the admission of
-// 9001 tokens (8 heads, 20 % admitted, W 1024) took 73 us (count 4.6, plan
-// 5.4, scatter 63.8); it takes 12 us in this form.
+// 9001 tokens (8 heads, 20 % admitted, W 1024) took 76 us in a trace (count
+// 4.6, plan 7.5, scatter 64.0); it takes 16.2 (4.5, 4.5, 7.2) in this form.
 __global__ __launch_bounds__(kThreads) void admit_scatter_kernel(AdmitArgs a) {
   __shared__ int s_src[kRows];
   __shared__ int s_w[kThreads / 64];

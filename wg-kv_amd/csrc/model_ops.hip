@@ -182,8 +182,8 @@ struct RopeArgs {
 // A token's threads are whole workgroups (or a workgroup holds whole tokens),
 // so a thread divides 32-bit indices only; with the hardware's bf16 conversions
 // the launch is bound by memory: 4096 tokens of 32 + 2 x 8 heads of 128 (100
-// MB) 28.0 us with 64-bit divisions and roundings in integer arithmetic, 19.7
-// us (5.1 TB/s) in this form.  PAD: heads padded to a power of two threads (a
+// MB), launched back to back, 28.0 us with 64-bit divisions and roundings in
+// integer arithmetic, 18.8 us (5.4 TB/s) in this form.  PAD: heads padded to a power of two threads (a
 // norm over 48, 80, 96, ... values), an instance of its own because the
 // padding's early returns keep the cos / sin loads from going out with the
 // rows': 64 + 2 x 8 heads of 128 took 30.1 us instead of 28.1.

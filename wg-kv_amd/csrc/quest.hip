@@ -87,7 +87,8 @@ struct SelectArgs {
 // pages, two of them per lane group in flight.  Bound by latency
 // (a 128K prompt's 13.1K pages are 6.7 MB of bounds): the group size is a
 // template argument, as a runtime bound put the per-member sums in scratch
-// memory and read the queries from LDS value by value (30 us; now 6.2 us).
+// memory and read the queries from LDS value by value (30.2 us, median of a
+// trace; now 6.8).
 template <int G, bool BF16>
 __global__ __launch_bounds__(kThreads) void quest_scores_kernel(SelectArgs a) {
   __shared__ __attribute__((aligned(16))) uint16_t s_q[G][256];
@@ -339,9 +340,9 @@ __device__ void select_few_pages(const float* sc, int full, int keep, const int3
 
 // One workgroup per head.  Bound by latency (a few memory round trips and the
 // steps' barriers); four waves rather than sixteen, whose barriers and scalar
-// counting cost more than the keys.  1638 pages per head, 8 heads: 15.0 us
-// with four LDS-histogram passes over the scores in memory, 8.1 us in this
-// form.
+// counting cost more than the keys.  1638 pages per head, 8 heads, bf16 scores,
+// medians of a trace: 14.7 us with four LDS-histogram passes over the scores in
+// memory, 9.0 us in this form.
 template <bool BF16>
 __global__ __launch_bounds__(kThreads) void quest_select_kernel(SelectArgs a) {
   __shared__ __attribute__((aligned(16))) uint32_t s_key[kMaxKeys];

@@ -570,7 +570,8 @@ hipError_t launch(const PrefillArgs& a, hipStream_t st, bool chunked) {
 // that two waves share -- unless the items are long: then loading a tile for
 // half of the heads costs more than the SIMD's second wave.  `reach` is the
 // last position, which bounds the tiles of an item; microseconds of 4 / 2 / 1
-// heads per workgroup, W 1024 and 20 % admitted unless said:
+// heads per workgroup, launched back to back, W 1024 and 20 % admitted unless
+// said:
 //   4 to 2 heads at any length for D 64 (one-shot, 1 KV head, G 4, 8000 tokens
 //   51.2 / 48.1 / 50.0; a 1024-token chunk at 131072, 8 KV heads, G 4, W 128 499
 //   / 489 / 640) and up to kLongReach for D 128 (one-shot, 8 KV heads, G 4: 500

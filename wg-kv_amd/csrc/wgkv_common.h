@@ -177,7 +177,7 @@ WGKV_DEVICE int count_flags(const uint8_t* m, int lo, int hi, int t, int n) {
 // Copies rows r < n of one K/V pair (source row src(r), pool row dst(r)) with
 // the whole workgroup of kThreads, 16 bytes per thread and step.  Eight loads per thread
 // are requested before the first store: one load and one store at a time
-// waited for memory once per step (64 us of a 9001-token prompt's 75).
+// waited for memory once per step (64 us of a 9001-token prompt's 76).
 template <int kThreads, typename Src, typename Dst>
 WGKV_DEVICE void copy_rows2(const uint16_t* ka, const uint16_t* va, int64_t ss, int n, int D, Src src, Dst dst,
                             uint16_t* pool_k, uint16_t* pool_v) {
